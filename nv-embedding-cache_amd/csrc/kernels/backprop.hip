@@ -121,7 +121,6 @@ __global__ __launch_bounds__(kPieceThreads) void piece_pool_kernel(PieceArgs a) 
   constexpr int U = BLK < 16 ? BLK : 16;
   constexpr int NB = BLK / U;
   const int lane = threadIdx.x & (G - 1);
-  const int wlane = threadIdx.x & 63;  // lane in the wave (the lane moves select by it)
   const int64_t b = (int64_t)blockIdx.x * kGroups + threadIdx.x / G;
   const int64_t p0 = b * BLK;
   if (p0 >= a.n) return;
@@ -144,15 +143,15 @@ __global__ __launch_bounds__(kPieceThreads) void piece_pool_kernel(PieceArgs a) 
   auto key_at = [&](auto I) -> uint32_t {
     constexpr int i = decltype(I)::value;
     if constexpr (i == BLK) return next_key;
-    else return group_bcast<G, i % G>(key[i / G], wlane);
+    else return group_bcast<G, i % G>(key[i / G]);
   };
   auto row_at = [&](auto I) -> uint32_t {
     constexpr int i = decltype(I)::value;
-    return group_bcast<G, i % G>(row[i / G], wlane);
+    return group_bcast<G, i % G>(row[i / G]);
   };
   auto wt_at = [&](auto I) -> float {
     constexpr int i = decltype(I)::value;
-    return __uint_as_float(group_bcast<G, i % G>(__float_as_uint(wt[i / G]), wlane));
+    return __uint_as_float(group_bcast<G, i % G>(__float_as_uint(wt[i / G])));
   };
   for (int c0 = 0; c0 < a.dim; c0 += G * V) {
     const int col = c0 + lane * V;

@@ -47,19 +47,18 @@ __device__ __forceinline__ void row_next_pin(uint32_t (&v)[4], const uint32_t (&
   v[3] = r3;
 }
 
-// Value of lane J of this lane's G-lane group (groups aligned to G lanes);
-// `lane` is this lane's index in the wave (0..63).
+// Value of lane J of this lane's G-lane group (groups aligned to G lanes).
 template <int G, int J>
-__device__ __forceinline__ uint32_t group_bcast(uint32_t v, int lane) {
+__device__ __forceinline__ uint32_t group_bcast(uint32_t v) {
   static_assert(J >= 0 && J < G, "broadcast source outside the group");
   if constexpr (G == 64) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, J);
   } else if constexpr (G == 16) {
     return dpp_mov<kDppRowNewBcast + J>(v);
   } else if constexpr (G == 8) {
+    // lane J to the whole row, then lane 8 + J to its lanes 8..15 (banks 2 and 3)
     const uint32_t lo = dpp_mov<kDppRowNewBcast + J>(v);
-    const uint32_t hi = dpp_mov<kDppRowNewBcast + 8 + J>(v);
-    return (lane & 8) ? hi : lo;
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)lo, (int)v, kDppRowNewBcast + 8 + J, 0xf, 0xc, false);
   } else {  // G == 32: lane J % 16 of each row, then the even or odd row of each pair
     static_assert(G == 32, "group of 8, 16, 32 or 64 lanes");
     const uint32_t b = dpp_mov<kDppRowNewBcast + (J & 15)>(v);

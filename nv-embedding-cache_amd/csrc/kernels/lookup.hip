@@ -587,6 +587,23 @@ hipError_t launch_gather(const GatherLaunch& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+int pool_groups_per_bag(const PoolLaunch& a, int g) {
+  const int64_t bags = a.num_bags;
+  const int64_t avg = a.keys_per_bag > 0 ? a.keys_per_bag : (bags > 0 ? a.num_keys / bags : 0);
+  int gpb = 1;
+  if (a.force_split > 0) {
+    gpb = pow2_ceil(a.force_split);
+  } else if (a.force_split == 0) {
+    // split long bags when there are too few bags to keep the chip's 256 CUs
+    // streaming: aim at ~16 keys per group, at least a whole wave per bag
+    if (avg > 32 && bags * (int64_t)g < 256LL * 1024) {
+      const int64_t want = avg / 16;
+      while ((int64_t)gpb * 2 <= want || gpb * g < 64) gpb <<= 1;
+    }
+  }
+  return gpb * g > 1024 ? 1024 / g : gpb;
+}
+
 bool pool_geometry(const PoolLaunch& a, PoolGeometry* g) {
   const int esize = value_elem_bytes(a.stored_dtype);
   const int64_t area = a.count * esize;
@@ -608,20 +625,7 @@ bool pool_geometry(const PoolLaunch& a, PoolGeometry* g) {
   const int passes = (int)((nv + G - 1) / G);
   const int64_t bags = a.num_bags;
   const int64_t avg = a.keys_per_bag > 0 ? a.keys_per_bag : (bags > 0 ? a.num_keys / bags : 0);
-  int gpb = 1;
-  if (a.force_split > 0) {
-    gpb = pow2_ceil(a.force_split);
-  } else if (a.force_split == 0) {
-    // split long bags when there are too few bags to keep the chip's 256 CUs
-    // streaming: aim at ~16 keys per group
-    if (avg > 32 && bags * (int64_t)G < 256LL * 1024) {
-      int64_t want = avg / 16;
-      gpb = 1;
-      while ((int64_t)gpb * 2 <= want) gpb <<= 1;
-    }
-  }
-  if (gpb * G > 1024) gpb = 1024 / G;
-  if (gpb < 1) gpb = 1;
+  const int gpb = pool_groups_per_bag(a, G);
   int threads;
   if (gpb == 1) {
     threads = 256;
@@ -649,11 +653,11 @@ bool pool_geometry(const PoolLaunch& a, PoolGeometry* g) {
 
 hipError_t launch_pool(const PoolLaunch& a, hipStream_t stream) {
   if (a.num_bags <= 0) return hipSuccess;
+  PoolSlices sl;
+  if (a.force_unroll == 0 && pool_slices(a, &sl)) return launch_pool_slices(a, sl, stream);
   PoolGeometry g;
   if (!pool_geometry(a, &g)) return hipErrorInvalidValue;
   if (g.grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  if (a.force_unroll == 0 && pool_split_eligible(a, g)) return launch_pool_split(a, g, stream);
-  if (a.force_unroll == 0 && pool_short_eligible(a, g)) return launch_pool_short(a, g, stream);
   switch (a.stored_dtype) {
     case kF32:
     case kF16:
