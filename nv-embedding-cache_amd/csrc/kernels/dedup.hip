@@ -599,7 +599,7 @@ hipError_t launch_hash_dedup_gather(const void* keys, int key_bytes, int64_t n, 
   return hipGetLastError();
 }
 
-int64_t dedup_span_parts(int64_t n) { return radix_tiles(n); }
+int64_t dedup_span_parts(int64_t n) { return radix_span_parts(n); }
 
 hipError_t launch_dedup_prep(const void* keys, int key_bytes, int64_t n, int flip, uint64_t* k64,
                              uint32_t* v, hipStream_t stream) {

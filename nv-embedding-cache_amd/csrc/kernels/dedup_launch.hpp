@@ -9,7 +9,7 @@
 namespace nve_amd {
 
 // Words of the key-span parts the radix sort's first pass writes for n keys
-// (one per tile, radix_tiles(n)).
+// (one per tile, radix_span_parts(n)).
 int64_t dedup_span_parts(int64_t n);
 // k64[i] = key i as an unsigned sort key (sign bit flipped when flip != 0), v[i] = i.
 hipError_t launch_dedup_prep(const void* keys, int key_bytes, int64_t n, int flip, uint64_t* k64,

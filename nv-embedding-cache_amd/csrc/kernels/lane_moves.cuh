@@ -67,6 +67,20 @@ __device__ __forceinline__ uint32_t group_bcast(uint32_t v) {
   }
 }
 
+// Inclusive sum over the 64 lanes of a wave (every lane on): shifts inside the
+// 16-lane rows, then each row's last lane to the rows after it.
+__device__ __forceinline__ uint32_t wave_sum_scan(uint32_t v) {
+  constexpr int kShr = 0x110, kBcast15 = 0x142, kBcast31 = 0x143;  // row_shr:n, row_bcast:15 / :31
+  // lanes without a source add the old value, 0
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kShr + 1, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kShr + 2, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kShr + 4, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kShr + 8, 0xf, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kBcast15, 0xa, 0xf, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kBcast31, 0xc, 0xf, false);
+  return v;
+}
+
 // f(integral_constant<int, b * U>) for b = B .. NB - 1, unrolled at compile time
 template <int U, int B, int NB, typename F>
 __device__ __forceinline__ void for_batches(F& f) {

@@ -8,35 +8,54 @@
 // Only the mathematical results matter (a stable sort; descending sorts are
 // expressed by the caller as ascending sorts of a complemented key).
 //
-// One pass per digit of 8 bits, or of 9 when that takes fewer passes (the
-// last digit keeps only the bits below end_bit), three kernels per pass:
-//   hist     each 256-thread workgroup counts the digits of its 1024-key tile
-//            into LDS and writes the counts digit-major;
-//   rowscan  one workgroup per digit turns its row of per-tile counts into
-//            exclusive prefixes (a separate array) and writes the digit's total;
-//   scatter  each workgroup scans the digit totals (digit d starts after
-//            every smaller digit) and adds its tile's row prefix (digit d of
-//            tile t lands after digit d of tiles < t: this is what makes the
-//            pass stable).  It ranks its keys stably inside the tile -- a wave
-//            finds the lanes sharing its digit with one ballot per digit bit, ranks by
-//            popcount of the lower lanes, and adds the counts of earlier waves
-//            and rounds -- stages the tile in LDS in digit order, and writes
-//            it out so that consecutive threads store consecutive positions of
-//            a digit's run.
+// One launch counts every digit of every pass (the digit counts of a pass do
+// not depend on the order of the keys), then one launch per pass moves the
+// keys.  Digits have 8 bits, or 9 when that takes fewer passes (the last digit
+// keeps only the bits below end_bit).
+//   count    at most kCountGroups workgroups, each the digit counts of its
+//            4096-key tiles for every pass; it also clears the passes' state;
+//   sweep    a 1024-thread workgroup per 4096-key tile.  A wave ranks its 256
+//            keys with one ballot per digit bit and a running count per digit
+//            in LDS; the tile's counts are published, the tile is staged in LDS
+//            in digit order, and each digit's place is found from the tiles
+//            before: their published counts are added, walking back until one
+//            that already knows its own place.  Consecutive threads then store
+//            consecutive positions of a digit's run.
+// A tile is numbered by a counter that its workgroup increments when it starts,
+// so the tiles it waits for have started before it, and every wait ends.  A
+// published word holds count and state together (one 64-bit store), so no other
+// memory has to be ordered against it.
 //
-// The exclusive scan of an array (run heads in dedup and insert) is
+// Bound: latency (a pass moves 24 bytes a key, 6 MB at 262,144 keys).  Three
+// launches per pass (tile counts, a scan of each digit's row, the scatter) took
+// NVE_OLD us of kernels for three passes over 262,144 keys, and nine launches; the
+// four take NVE_NEW.  The tile is 4096 keys so that a tile has few predecessors:
+// with 1024-key tiles every one of 256 tiles walks back through most of them.
+//
+// The exclusive scan of an array (run heads in the insert) is
 // reduce-then-scan over 4096-element blocks: block sums, a scan of the sums
 // (recursively, in the caller's temporary storage), then each block rescans
 // its elements from its offset.
 #include "device_common.cuh"
+#include "lane_moves.cuh"
 #include "sort_launch.hpp"
 
 namespace nve_amd {
 
-constexpr int kSortThreads = 256;
-constexpr int kSortItems = 4;
-constexpr int kSortTile = kSortThreads * kSortItems;
-constexpr int kMaxBins = 512;  // digits of at most 9 bits
+constexpr int kTileThreads = 1024;
+constexpr int kTileWaves = kTileThreads / 64;
+constexpr int kTileItems = 4;  // rounds of 64 keys per wave
+constexpr int kTile = kTileThreads * kTileItems;
+constexpr int kMaxBins = 512;     // digits of at most 9 bits
+constexpr int kMaxPasses = 8;     // 64 bits in digits of 8, or of 9
+constexpr int kCountGroups = 64;  // workgroups whose digit counts every tile adds up
+
+// The digits of a sort: pass p takes (key >> shift[p]) & mask[p].
+struct RadixDigits {
+  int passes;
+  int shift[kMaxPasses];
+  uint32_t mask[kMaxPasses];
+};
 
 // The sort key of position i: keys[i], or with a raw source the caller's key
 // converted on the fly (sign bit flipped when src.flip).
@@ -50,48 +69,70 @@ __device__ __forceinline__ uint64_t sort_key(const uint64_t* keys, const RadixSo
   }
 }
 
-// RAW: the first pass over the caller's keys; with src.span_part, also the
-// tile's OR of key ^ key[0] (the bits where its keys differ from the first).
-template <int RB, bool RAW>
-__global__ __launch_bounds__(256) void radix_hist_kernel(const uint64_t* keys, RadixSource src, int64_t n,
-                                                         int shift, uint32_t mask, uint32_t* counts,
-                                                         int nblocks) {
-  constexpr int kBins = 1 << RB;
-  __shared__ uint32_t h[kBins];
+// parts[workgroup][pass][kMaxBins] = digit counts of the workgroup's tiles;
+// state[0 .. state_words) = 0.  With src.span_part, span_part[workgroup] = the
+// OR of key ^ key[0] over its keys (the bits where they differ from the first).
+template <bool RAW>
+__global__ __launch_bounds__(kTileThreads) void radix_count_kernel(const uint64_t* keys, RadixSource src,
+                                                                   int64_t n, RadixDigits dg, uint32_t* parts,
+                                                                   uint64_t* state, int64_t state_words) {
+  __shared__ uint32_t h[kMaxPasses * kMaxBins];
   const int tid = threadIdx.x;
-#pragma unroll
-  for (int d = tid; d < kBins; d += kSortThreads) h[d] = 0;
+  for (int64_t w = (int64_t)blockIdx.x * kTileThreads + tid; w < state_words; w += (int64_t)gridDim.x * kTileThreads)
+    state[w] = 0;
+  for (int d = tid; d < dg.passes * kMaxBins; d += kTileThreads) h[d] = 0;
   __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * kSortTile;
   uint64_t diff = 0;
-  const uint64_t k0 = RAW && src.span_part != nullptr ? sort_key<RAW>(keys, src, 0) : 0;
+  const uint64_t k0 = sort_key<RAW>(keys, src, 0);
+  for (int64_t base = (int64_t)blockIdx.x * kTile; base < n; base += (int64_t)gridDim.x * kTile) {
+    uint64_t k[kTileItems];
 #pragma unroll
-  for (int r = 0; r < kSortItems; ++r) {
-    const int64_t i = base + r * kSortThreads + tid;
-    if (i < n) {
-      const uint64_t k = sort_key<RAW>(keys, src, i);
-      atomicAdd(&h[(uint32_t)(k >> shift) & mask], 1u);
-      diff |= k ^ k0;
+    for (int r = 0; r < kTileItems; ++r) {
+      const int64_t i = base + r * kTileThreads + tid;
+      k[r] = sort_key<RAW>(keys, src, i < n ? i : 0);
     }
-  }
-  if constexpr (RAW) {
-    if (src.span_part != nullptr) {  // uniform
 #pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) diff |= __shfl_xor(diff, o);
-      __shared__ uint64_t red[kSortThreads / 64];
-      if ((tid & 63) == 0) red[tid >> 6] = diff;
-      __syncthreads();
-      if (tid == 0) {
-        uint64_t x = 0;
-#pragma unroll
-        for (int w = 0; w < kSortThreads / 64; ++w) x |= red[w];
-        src.span_part[blockIdx.x] = x;
+    for (int r = 0; r < kTileItems; ++r) {
+      const bool valid = base + r * kTileThreads + tid < n;
+      diff |= k[r] ^ k0;  // a lane past the end holds key 0
+      for (int p = 0; p < dg.passes; ++p) {
+        // the digit of the wave's first lane is added once for all lanes that
+        // share it: a hot key's (or a high digit's) lanes would queue on its word
+        const uint32_t d = (uint32_t)(k[r] >> dg.shift[p]) & dg.mask[p];
+        const uint32_t lead = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
+        const uint64_t same = __ballot(valid && d == lead);
+        if (valid && d != lead) atomicAdd(&h[p * kMaxBins + d], 1u);
+        if ((tid & 63) == 0 && same) atomicAdd(&h[p * kMaxBins + lead], (uint32_t)__popcll(same));
       }
     }
   }
-  __syncthreads();
+  if (src.span_part != nullptr) {  // uniform
 #pragma unroll
-  for (int d = tid; d < kBins; d += kSortThreads) counts[(int64_t)d * nblocks + blockIdx.x] = h[d];
+    for (int o = 32; o >= 1; o >>= 1) diff |= __shfl_xor(diff, o);
+    __shared__ uint64_t red[kTileWaves];
+    if ((tid & 63) == 0) red[tid >> 6] = diff;
+    __syncthreads();
+    if (tid == 0) {
+      uint64_t x = 0;
+#pragma unroll
+      for (int w = 0; w < kTileWaves; ++w) x |= red[w];
+      src.span_part[blockIdx.x] = x;
+    }
+  }
+  __syncthreads();
+  uint32_t* out = parts + (int64_t)blockIdx.x * dg.passes * kMaxBins;
+  for (int d = tid; d < dg.passes * kMaxBins; d += kTileThreads) out[d] = h[d];
+}
+
+// parts[0] = the sum of parts[0 .. nparts): with many tiles, each adding up
+// nparts counts would cost more than this launch.
+__global__ __launch_bounds__(256) void radix_total_kernel(uint32_t* parts, int nparts, int stride) {
+  const int d = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (d >= stride) return;
+  uint32_t t = 0;
+#pragma unroll 16
+  for (int w = 0; w < nparts; ++w) t += parts[(int64_t)w * stride + d];
+  parts[d] = t;
 }
 
 // Inclusive scan across the 64 lanes of a wave.
@@ -174,154 +215,187 @@ __global__ __launch_bounds__(256) void scan_down_kernel(uint32_t* data, int64_t 
     *total = off + block_total;
 }
 
-// Exclusive scan of the D consecutive values v[0..D) of each of the
-// workgroup's NT threads (thread t holds items t*D .. t*D+D-1), in place.
-template <int NT, int D>
-__device__ __forceinline__ void block_exclusive_scan_items(uint32_t* v, uint32_t* lds,
-                                                           uint32_t* total) {
-  uint32_t s = 0;
+// A published word: state in the top two bits, a count of keys below.
+constexpr uint64_t kStateOwn = 1ull << 62;     // the tile's own keys of the digit
+constexpr uint64_t kStateBefore = 2ull << 62;  // with those of every tile before it
+constexpr uint64_t kStateCount = (1ull << 62) - 1;
+constexpr int kLookAhead = 8;  // words read at a time while walking back
+
+// Keys of the tiles before `tile`, from word[tile * stride]: adds published
+// counts from tile - 1 down until one that includes all before it.
+__device__ __forceinline__ uint64_t keys_before(const uint64_t* word, int64_t tile, int64_t stride) {
+  uint64_t sum = 0;
+  for (int64_t j = tile - 1; j >= 0;) {
+    uint64_t w[kLookAhead];
 #pragma unroll
-  for (int j = 0; j < D; ++j) s += v[j];
-  uint32_t run = block_exclusive_scan<NT>(s, lds, total);
+    for (int u = 0; u < kLookAhead; ++u)
+      w[u] = j - u >= 0 ? __hip_atomic_load(word + (j - u) * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                        : kStateBefore;  // nothing before the first tile
+    bool open = true;  // every word so far was published, none of them the last to add
+    int used = 0;
 #pragma unroll
-  for (int j = 0; j < D; ++j) {
-    const uint32_t x = v[j];
-    v[j] = run;
-    run += x;
+    for (int u = 0; u < kLookAhead; ++u) {
+      if (open && w[u] >= kStateOwn) {
+        sum += w[u] & kStateCount;
+        ++used;
+        if (w[u] >= kStateBefore) return sum;
+      } else {
+        open = false;
+      }
+    }
+    j -= used;
+    if (used == 0) __builtin_amdgcn_s_sleep(1);
   }
+  return sum;
 }
 
-// Row d of the digit-major per-tile counts -> exclusive prefixes in offs;
-// totals[d] = the row's sum.  One workgroup per digit.
-__global__ __launch_bounds__(256) void radix_rowscan_kernel(const uint32_t* counts, uint32_t* offs,
-                                                            int nblocks, uint32_t* totals) {
-  __shared__ uint32_t lds[256 / 64 + 1];
-  const uint32_t* row = counts + (int64_t)blockIdx.x * nblocks;
-  uint32_t* orow = offs + (int64_t)blockIdx.x * nblocks;
-  uint32_t carry = 0;
-  for (int c = 0; c < nblocks; c += 256 * 4) {
-    const int b = c + (int)threadIdx.x * 4;
-    uint32_t v[4];
-    uint32_t s = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[j] = b + j < nblocks ? row[b + j] : 0u;
-      s += v[j];
-    }
-    uint32_t chunk_total;
-    uint32_t run = carry + block_exclusive_scan<256>(s, lds, &chunk_total);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (b + j < nblocks) orow[b + j] = run;
-      run += v[j];
-    }
-    carry += chunk_total;
-  }
-  if (threadIdx.x == 0) totals[blockIdx.x] = carry;
-}
+struct SweepArgs {
+  const uint64_t* keys;
+  const uint32_t* vals;
+  RadixSource src;  // RAW: the first pass reads the caller's keys, values = positions
+  uint64_t* ko;
+  uint32_t* vo;
+  int64_t n;
+  int shift;
+  uint32_t mask;
+  const uint32_t* parts;  // the pass's digit counts, nparts of them part_stride apart
+  int nparts;
+  int part_stride;
+  uint64_t* state;  // the pass's words: tile counter, then kMaxBins per tile
+};
 
-// RAW: the first pass reads the caller's keys (src) and takes each key's
-// position as its value.
 template <int RB, bool RAW>
-__global__ __launch_bounds__(256) void radix_scatter_kernel(const uint64_t* keys, const uint32_t* vals,
-                                                            RadixSource src, uint64_t* ko, uint32_t* vo,
-                                                            int64_t n, int shift, uint32_t mask,
-                                                            const uint32_t* counts,
-                                                            const uint32_t* offs,
-                                                            const uint32_t* totals, int nblocks) {
+__global__ __launch_bounds__(kTileThreads) void radix_sweep_kernel(SweepArgs a) {
   constexpr int kBins = 1 << RB;
-  constexpr int D = kBins / kSortThreads;                    // digits per thread
-  constexpr int kSlots = kSortItems * (kSortThreads / 64);  // (round, wave) pairs in key order
-  __shared__ uint64_t sk[kSortTile];
-  __shared__ uint32_t sv[kSortTile];
-  __shared__ uint32_t lstart[kBins];          // first local position of digit d in the tile
-  __shared__ uint32_t gbase[kBins];           // output position of that key
-  __shared__ uint32_t slot[kSlots][kBins];    // keys of digit d per (round, wave), then their prefix
-  __shared__ uint32_t lds[256 / 64 + 1];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int64_t base = (int64_t)blockIdx.x * kSortTile;
-  const int tile_n = (int)(n - base < kSortTile ? n - base : kSortTile);
-  // all of the tile's loads in flight at once
-  uint64_t k[kSortItems];
-  uint32_t v[kSortItems];
+  static_assert(kBins <= kTileThreads && kBins <= kMaxBins, "one thread per digit");
+  __shared__ uint64_t sk[kTile];
+  __shared__ uint32_t sv[kTile];
+  __shared__ uint32_t cnt[kTileWaves][kBins];  // keys of digit d per wave, then of the waves before
+  __shared__ uint32_t lstart[kBins];           // first position of digit d in the staged tile
+  __shared__ uint32_t gbase[kBins];            // output position of staged position 0, were it digit d's
+  __shared__ uint64_t scan[kTileWaves + 1];
+  __shared__ uint32_t s_tile;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (tid == 0) s_tile = (uint32_t)atomicAdd(reinterpret_cast<unsigned long long*>(a.state), 1ull);
+  // the keys of tile blockIdx.x, which mostly is the tile: loaded while the
+  // counter's answer is on its way
+  const int li0 = wave * (64 * kTileItems) + lane;  // key r of the lane: li0 + 64 * r
+  uint64_t k[kTileItems];
+  uint32_t v[kTileItems];
+  int tile_n;
+  const auto load = [&](int64_t t) {
+    const int64_t base = t * kTile;
+    tile_n = (int)(a.n - base < kTile ? a.n - base : kTile);
 #pragma unroll
-  for (int r = 0; r < kSortItems; ++r) {
-    const int li = r * kSortThreads + tid;
-    k[r] = li < tile_n ? sort_key<RAW>(keys, src, base + li) : 0ull;
-    if constexpr (RAW)
-      v[r] = (uint32_t)(base + li);
-    else
-      v[r] = li < tile_n ? vals[base + li] : 0u;
+    for (int r = 0; r < kTileItems; ++r) {
+      const int li = li0 + 64 * r;
+      k[r] = li < tile_n ? sort_key<RAW>(a.keys, a.src, base + li) : 0ull;
+      if constexpr (RAW)
+        v[r] = (uint32_t)(base + li);
+      else
+        v[r] = li < tile_n ? a.vals[base + li] : 0u;
+    }
+  };
+  load(blockIdx.x);
+  // the pass's total of digit tid % kBins, from every kAdders-th part
+  constexpr int kAdders = kTileThreads / kBins;
+  constexpr int kLoads = kCountGroups / kAdders;
+  uint32_t total = 0;
+  {
+    uint32_t c[kLoads];
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      const int w = u * kAdders + tid / kBins;
+      c[u] = w < a.nparts ? a.parts[(int64_t)w * a.part_stride + (tid & (kBins - 1))] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) total += c[u];
   }
-  // thread t owns digits t*D .. t*D+D-1
-  uint32_t dbase[D], loc[D];
-#pragma unroll
-  for (int j = 0; j < D; ++j) {
-    const int d = tid * D + j;
-    dbase[j] = totals[d];
-    loc[j] = counts[(int64_t)d * nblocks + blockIdx.x];
-  }
-  uint32_t all;
-  block_exclusive_scan_items<kSortThreads, D>(dbase, lds, &all);
-  block_exclusive_scan_items<kSortThreads, D>(loc, lds, &all);
-#pragma unroll
-  for (int j = 0; j < D; ++j) {
-    const int d = tid * D + j;
-    lstart[d] = loc[j];
-    gbase[d] = dbase[j] + offs[(int64_t)d * nblocks + blockIdx.x];
-#pragma unroll
-    for (int q = 0; q < kSlots; ++q) slot[q][d] = 0;
-  }
+  for (int d = tid; d < kTileWaves * kBins; d += kTileThreads) (&cnt[0][0])[d] = 0;
+  sv[tid] = total;
   __syncthreads();
-  // per (round, wave): lanes sharing the digit, rank among them, count by the leader
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  uint32_t rank[kSortItems];
+  if (tid < kBins) {
 #pragma unroll
-  for (int r = 0; r < kSortItems; ++r) {
-    const bool valid = r * kSortThreads + tid < tile_n;
-    const uint32_t d = (uint32_t)(k[r] >> shift) & mask;
-    uint64_t peers = __ballot(valid);
+    for (int q = 1; q < kAdders; ++q) total += sv[q * kBins + tid];
+  } else {
+    total = 0;
+  }
+  const int64_t tile = s_tile;
+  if (tile != blockIdx.x) load(tile);  // uniform
+  // rank among the wave's keys of the same digit: earlier rounds, then lower lanes
+  const uint64_t lower = (1ull << lane) - 1ull;
+  uint32_t rank[kTileItems];
+#pragma unroll
+  for (int r = 0; r < kTileItems; ++r) {
+    const bool valid = li0 + 64 * r < tile_n;
+    const uint32_t d = (uint32_t)(k[r] >> a.shift) & a.mask;
+    const uint64_t valids = __ballot(valid);
+    uint32_t plo = (uint32_t)valids, phi = (uint32_t)(valids >> 32);
 #pragma unroll
     for (int b = 0; b < RB; ++b) {
       const uint64_t m = __ballot((d >> b) & 1u);
-      peers &= ((d >> b) & 1u) ? m : ~m;
+      const uint32_t mine = 0u - ((d >> b) & 1u);  // lanes whose bit differs leave
+      plo &= ~((uint32_t)m ^ mine);
+      phi &= ~((uint32_t)(m >> 32) ^ mine);
     }
-    rank[r] = (uint32_t)__popcll(peers & lt_mask);
-    if (valid && rank[r] == 0) slot[r * (kSortThreads / 64) + wave][d] = (uint32_t)__popcll(peers);
+    const uint64_t peers = ((uint64_t)phi << 32) | plo;
+    const uint32_t before = (uint32_t)__popcll(peers & lower);
+    // a wave's LDS accesses stay in order: every lane reads the count before
+    // the first of its digit's lanes adds to it
+    const uint32_t seen = cnt[wave][d];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (valid && before == 0) cnt[wave][d] = seen + (uint32_t)__popcll(peers);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    rank[r] = seen + before;
   }
   __syncthreads();
-  // digit d: exclusive prefix over the slots, from its local start
+  uint64_t* const word = a.state + 1 + (tid < kBins ? tid : 0);
+  uint32_t own = 0;
+  if (tid < kBins) {
 #pragma unroll
-  for (int j = 0; j < D; ++j) {
-    const int d = tid * D + j;
-    uint32_t acc = lstart[d];
-#pragma unroll
-    for (int q = 0; q < kSlots; ++q) {
-      const uint32_t c = slot[q][d];
-      slot[q][d] = acc;
-      acc += c;
+    for (int w = 0; w < kTileWaves; ++w) {
+      const uint32_t c = cnt[w][tid];
+      cnt[w][tid] = own;
+      own += c;
     }
+    __hip_atomic_store(word + tile * kMaxBins, (tile == 0 ? kStateBefore : kStateOwn) | own, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
   }
+  // exclusive sums over the digits: the tile's counts and the totals
+  const uint32_t inc_own = wave_sum_scan(own), inc_total = wave_sum_scan(total);
+  if (lane == 63) scan[wave] = ((uint64_t)inc_total << 32) | inc_own;
+  __syncthreads();
+  uint64_t ex = ((uint64_t)(inc_total - total) << 32) | (inc_own - own);
+#pragma unroll
+  for (int w = 0; w < kBins / 64; ++w)
+    if (w < wave) ex += scan[w];
+  if (tid < kBins) lstart[tid] = (uint32_t)ex;
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kSortItems; ++r) {
-    if (r * kSortThreads + tid < tile_n) {
-      const uint32_t d = (uint32_t)(k[r] >> shift) & mask;
-      const uint32_t pos = slot[r * (kSortThreads / 64) + wave][d] + rank[r];
+  for (int r = 0; r < kTileItems; ++r) {
+    if (li0 + 64 * r < tile_n) {
+      const uint32_t d = (uint32_t)(k[r] >> a.shift) & a.mask;
+      const uint32_t pos = lstart[d] + cnt[wave][d] + rank[r];
       sk[pos] = k[r];
       sv[pos] = v[r];
     }
   }
+  if (tid < kBins) {
+    const uint64_t before = keys_before(word, tile, kMaxBins);
+    if (tile > 0)
+      __hip_atomic_store(word + tile * kMaxBins, kStateBefore | (before + own), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    gbase[tid] = (uint32_t)(ex >> 32) + (uint32_t)before - (uint32_t)ex;
+  }
   __syncthreads();
   // the tile in digit order: runs of one digit go to consecutive positions
-  for (int j = tid; j < tile_n; j += kSortThreads) {
+  for (int j = tid; j < tile_n; j += kTileThreads) {
     const uint64_t kk = sk[j];
-    const uint32_t d = (uint32_t)(kk >> shift) & mask;
-    const uint32_t pos = gbase[d] + (uint32_t)j - lstart[d];
-    ko[pos] = kk;
-    vo[pos] = sv[j];
+    const uint32_t pos = gbase[(uint32_t)(kk >> a.shift) & a.mask] + (uint32_t)j;
+    a.ko[pos] = kk;
+    a.vo[pos] = sv[j];
   }
 }
 
@@ -356,10 +430,18 @@ size_t scan_temp_bytes(int64_t m) {
   return bytes;
 }
 
+namespace {
+int64_t tiles_of(int64_t n) { return n > 0 ? (n + kTile - 1) / kTile : 1; }
+int64_t pass_words(int64_t n) { return 1 + tiles_of(n) * kMaxBins; }
+// past this many tiles one launch adds the counts up
+constexpr int64_t kMaxAddingTiles = 128;
+}  // namespace
+
+int64_t radix_span_parts(int64_t n) { return tiles_of(n) < kCountGroups ? tiles_of(n) : kCountGroups; }
+
 size_t radix_sort_temp_bytes(int64_t n) {
-  const int64_t nblocks = (n + kSortTile - 1) / kSortTile;
-  const size_t sort = (size_t)(nblocks > 0 ? nblocks : 1) * kMaxBins * sizeof(uint32_t) * 2 +
-                      kMaxBins * sizeof(uint32_t) + 1024;
+  const size_t sort = (size_t)kMaxPasses * (size_t)pass_words(n) * 8 +
+                      (size_t)radix_span_parts(n) * kMaxPasses * kMaxBins * 4;
   const size_t scan = scan_temp_bytes(n);
   return sort > scan ? sort : scan;
 }
@@ -369,56 +451,70 @@ hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, 
                             hipStream_t stream, const RadixSource* src) {
   *result_in_alt = 0;
   if (n <= 1 || end_bit <= begin_bit) return src != nullptr ? hipErrorInvalidValue : hipSuccess;
-  const int64_t nblocks = (n + kSortTile - 1) / kSortTile;
-  if (nblocks > 0x7fffffff) return hipErrorInvalidValue;
-  uint32_t* counts = static_cast<uint32_t*>(temp);
-  uint32_t* offs = counts + nblocks * kMaxBins;
-  uint32_t* totals = offs + nblocks * kMaxBins;
-  uint64_t* ki = keys;
-  uint32_t* vi = vals;
-  uint64_t* ka = keys_alt;
-  uint32_t* va = vals_alt;
-  const RadixSource none{};
+  if (n > 0xffffffffLL || end_bit > 64) return hipErrorInvalidValue;  // values and counts of 32 bits
+  const int64_t tiles = tiles_of(n);
   // 9-bit digits when they take fewer passes than 8-bit ones (26-bit keys: 3
-  // passes instead of 4); the last digit keeps only the bits below end_bit.
-  // (10-bit digits measured no better: three 10-bit passes over 262,144 keys
-  // took as long as four 8-bit ones, 17.4 against 13.1 us a pass.)
+  // passes instead of 4); the last digit keeps only the bits below end_bit
   const int width = end_bit - begin_bit;
   const int rb = (width + 8) / 9 < (width + 7) / 8 ? 9 : 8;
+  RadixDigits dg{};
   for (int shift = begin_bit; shift < end_bit; shift += rb) {
     const int bits = end_bit - shift < rb ? end_bit - shift : rb;
-    const uint32_t mask = (1u << bits) - 1u;
-    const bool raw = src != nullptr && shift == begin_bit;
-    const RadixSource& s = raw ? *src : none;
-#define NVE_RADIX_PASS(RB, RAW)                                                                           \
-  hipLaunchKernelGGL((radix_hist_kernel<RB, RAW>), dim3(nblocks), dim3(kSortThreads), 0, stream, ki, s, n, \
-                     shift, mask, counts, (int)nblocks);                                                  \
-  hipLaunchKernelGGL(radix_rowscan_kernel, dim3(1u << RB), dim3(256), 0, stream, counts, offs,            \
-                     (int)nblocks, totals);                                                               \
-  hipLaunchKernelGGL((radix_scatter_kernel<RB, RAW>), dim3(nblocks), dim3(kSortThreads), 0, stream, ki,   \
-                     vi, s, ka, va, n, shift, mask, counts, offs, totals, (int)nblocks)
+    dg.shift[dg.passes] = shift;
+    dg.mask[dg.passes] = (1u << bits) - 1u;
+    ++dg.passes;
+  }
+  uint64_t* state = static_cast<uint64_t*>(temp);
+  const int64_t words = pass_words(n);
+  uint32_t* parts = reinterpret_cast<uint32_t*>(state + (int64_t)dg.passes * words);
+  int nparts = (int)radix_span_parts(n);
+  const int stride = dg.passes * kMaxBins;
+  const RadixSource none{};
+  if (src != nullptr)
+    hipLaunchKernelGGL(radix_count_kernel<true>, dim3(nparts), dim3(kTileThreads), 0, stream, keys, *src, n, dg,
+                       parts, state, dg.passes * words);
+  else
+    hipLaunchKernelGGL(radix_count_kernel<false>, dim3(nparts), dim3(kTileThreads), 0, stream, keys, none, n, dg,
+                       parts, state, dg.passes * words);
+  if (tiles > kMaxAddingTiles) {
+    hipLaunchKernelGGL(radix_total_kernel, dim3((stride + 255) / 256), dim3(256), 0, stream, parts, nparts, stride);
+    nparts = 1;
+  }
+  SweepArgs a{};
+  a.keys = keys;
+  a.vals = vals;
+  a.ko = keys_alt;
+  a.vo = vals_alt;
+  a.n = n;
+  a.nparts = nparts;
+  a.part_stride = stride;
+  for (int p = 0; p < dg.passes; ++p) {
+    a.shift = dg.shift[p];
+    a.mask = dg.mask[p];
+    a.parts = parts + p * kMaxBins;
+    a.state = state + p * words;
+    const bool raw = src != nullptr && p == 0;
+    a.src = raw ? *src : none;
+    const dim3 grid((unsigned)tiles), block(kTileThreads);
     if (rb == 9) {
-      if (raw) {
-        NVE_RADIX_PASS(9, true);
-      } else {
-        NVE_RADIX_PASS(9, false);
-      }
+      if (raw)
+        hipLaunchKernelGGL((radix_sweep_kernel<9, true>), grid, block, 0, stream, a);
+      else
+        hipLaunchKernelGGL((radix_sweep_kernel<9, false>), grid, block, 0, stream, a);
     } else {
-      if (raw) {
-        NVE_RADIX_PASS(8, true);
-      } else {
-        NVE_RADIX_PASS(8, false);
-      }
+      if (raw)
+        hipLaunchKernelGGL((radix_sweep_kernel<8, true>), grid, block, 0, stream, a);
+      else
+        hipLaunchKernelGGL((radix_sweep_kernel<8, false>), grid, block, 0, stream, a);
     }
-#undef NVE_RADIX_PASS
-    std::swap(ki, ka);
-    std::swap(vi, va);
+    a.keys = p & 1 ? keys : keys_alt;
+    a.vals = p & 1 ? vals : vals_alt;
+    a.ko = p & 1 ? keys_alt : keys;
+    a.vo = p & 1 ? vals_alt : vals;
     *result_in_alt ^= 1;
   }
   return hipGetLastError();
 }
-
-int64_t radix_tiles(int64_t n) { return n > 0 ? (n + kSortTile - 1) / kSortTile : 0; }
 
 hipError_t exclusive_scan_u32(uint32_t* data, int64_t m, uint32_t* total, void* temp,
                               hipStream_t stream) {

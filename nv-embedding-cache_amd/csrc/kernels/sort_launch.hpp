@@ -16,15 +16,15 @@ size_t scan_temp_bytes(int64_t m);
 
 // The caller's keys as the first pass's input: keys of key_bytes bytes at
 // `keys` (sign bit flipped when flip != 0), values = positions; span_part
-// (optional, radix_tiles(n) words) receives each tile's OR of key ^ key[0].
+// (optional, radix_span_parts(n) words) receives ORs of key ^ key[0] whose OR is
+// that of all keys.
 struct RadixSource {
   const void* keys;
   int key_bytes;
   int flip;
   uint64_t* span_part;
 };
-// Tiles (workgroups) of one radix pass over n keys.
-int64_t radix_tiles(int64_t n);
+int64_t radix_span_parts(int64_t n);
 
 // Stable ascending sort of (keys[i], vals[i]) on bits [begin_bit, end_bit) of
 // the keys (digits of 8 or 9 bits from begin_bit).  Ping-pongs between (keys, vals) and

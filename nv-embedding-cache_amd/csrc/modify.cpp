@@ -208,11 +208,11 @@ void GpuTable::modify_insert(ExecutionContext& ctx, hipStream_t s, int64_t n, co
   // ---- scratch (grow-only, per context) ----
   const size_t un = (size_t)n;
   const size_t bytes = 18 * 256 + un * (8 * 2 + 4 * 2) * 3 + un * (4 * 4 + 8 * 4) +
-                       (size_t)radix_tiles(n) * 8 + radix_sort_temp_bytes(n) + 64 * 256;
+                       (size_t)radix_span_parts(n) * 8 + radix_sort_temp_bytes(n) + 64 * 256;
   uint8_t* p = static_cast<uint8_t*>(ctx.buffer("insert_scratch", bytes));
   unsigned long long* d_span = carve<unsigned long long>(p, 1);
   InsertHead* head = carve<InsertHead>(p, 1);
-  uint64_t* span_part = carve<uint64_t>(p, (size_t)radix_tiles(n));
+  uint64_t* span_part = carve<uint64_t>(p, (size_t)radix_span_parts(n));
   uint32_t* d_count = carve<uint32_t>(p, 4);
   uint64_t* ka = carve<uint64_t>(p, un);
   uint32_t* va = carve<uint32_t>(p, un);
@@ -240,7 +240,7 @@ void GpuTable::modify_insert(ExecutionContext& ctx, hipStream_t s, int64_t n, co
     // the first pass reads the caller's keys and writes each tile's span part
     const RadixSource src{d_keys, key_bytes_, 1, span_part};
     NVE_HIP(radix_sort_pairs(ka, va, kb, vb, n, 0, kInsertSpecBits, sort_tmp, &alt, s, &src));
-    NVE_HIP(launch_run_heads(alt ? kb : ka, n, heads, s, span_part, radix_tiles(n), &head->span));
+    NVE_HIP(launch_run_heads(alt ? kb : ka, n, heads, s, span_part, radix_span_parts(n), &head->span));
     NVE_HIP(exclusive_scan_u32(heads, n, &head->uniq, sort_tmp, s));
     const InsertHead h = read_back(head, s);
     exact = (h.span >> kInsertSpecBits) != 0;

@@ -1,0 +1,55 @@
+"""The radix sort behind the dedup at the sizes where its tiles change: one
+tile of 4,096 keys and one key more or less, the 64 count groups, the launch
+that adds counts up (beyond 128 tiles), and keys whose digits pile up in one
+bin, all equal, descending, or spread over all 64 bits."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from nve_helpers import stream_ptr, to_dev, vp
+from pynve import _lib
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+TILE = 4096
+
+
+def make(kind, n, rng):
+    if kind == "table":  # rows of a table: the 27-bit passes
+        return (rng.random(n) ** 4 * 5e7).astype(np.int64)
+    if kind == "wide":  # every bit, both signs: sorted again on the exact bits
+        return rng.integers(-2**63, 2**63 - 1, size=n, dtype=np.int64)
+    if kind == "one":
+        return np.full(n, 12345, np.int64)
+    if kind == "descending":
+        return np.arange(n, 0, -1).astype(np.int64)
+    hot = np.where(rng.random(n) < 0.9, 7, rng.integers(0, 1 << 20, size=n))
+    return hot.astype(np.int64)
+
+
+@pytest.mark.parametrize("kind", ["table", "wide", "one", "descending", "hot"])
+@pytest.mark.parametrize("n", [2, 63, 64, 65, TILE - 1, TILE, TILE + 1, 3 * TILE + 17, 63 * TILE + 1, 64 * TILE,
+                               65 * TILE + 5, 128 * TILE, 128 * TILE + 1, 300 * TILE + 9])
+def test_dedup_equals_numpy(kind, n):
+    if n > 65 * TILE + 5 and kind in ("wide", "descending"):
+        n = 129 * TILE + 3
+    rng = np.random.default_rng(n)
+    keys = make(kind, n, rng)
+    need = ctypes.c_uint64()
+    _lib.call("nve_amd_dedup_workspace_size", n, ctypes.byref(need))
+    ws = torch.full((need.value,), 0xEE, dtype=torch.uint8, device="cuda")
+    out = [torch.zeros(n + 1, dtype=torch.int64, device="cuda") for _ in range(4)]
+    num, d_keys = ctypes.c_int64(), to_dev(keys)
+    for _ in range(2):  # the second call finds the first one's state in its workspace
+        _lib.call("nve_amd_dedup", _lib.KEY_INT64, n, vp(d_keys), vp(out[0]), vp(out[1]), vp(out[2]), vp(out[3]),
+                  ctypes.byref(num), vp(ws), need.value, stream_ptr())
+        unique, start, counts = np.unique(keys, return_index=True, return_counts=True)
+        u = num.value
+        assert u == unique.size
+        got = [t.cpu().numpy() for t in out]
+        assert np.array_equal(got[0][:u], unique)
+        assert np.array_equal(got[1][:u], counts)
+        assert np.array_equal(got[2][:n], np.argsort(keys, kind="stable"))
+        assert np.array_equal(got[3][:u], np.cumsum(counts) - counts)
