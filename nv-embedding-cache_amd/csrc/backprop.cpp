@@ -3,10 +3,10 @@
 // cuda_ops/gradient_calculator.cuh:238-301, reached from pynve's
 // concat_backprop / pooling_backprop, python/pynve/bindings/binding_layers.hpp:131-250).
 //
-//   keys -> dedup (unique keys ascending, stable inverse, the unique index of
-//           every dedup position)                                  dedup.cpp
-//        -> per dedup position: the gradient row it reads (its bag, or
-//           its own position for Concatenate) and its weight        backprop.hip
+//   keys -> dedup (unique keys ascending, the unique index of every dedup
+//           position) and on the way, per dedup position, the gradient row it
+//           reads (its bag, or its own position for Concatenate) and its
+//           weight                                                  dedup.cpp
 //        -> piece_pool_kernel: each block of kPieceBlock dedup positions added
 //           per key in position order (fp32); keys inside a block finished
 //           there, pieces of keys crossing a block edge kept as fp32 rows and
@@ -36,8 +36,8 @@ size_t pad(size_t b) { return (b + 255) / 256 * 256; }
 struct BackpropBufs {
   uint8_t* dedup_ws;
   size_t dedup_bytes;
-  void *counts, *inverse, *doff;
-  uint32_t *kidx, *rows, *cross;
+  void *counts, *doff;
+  uint32_t *kidx, *rows, *by_key, *cross;
   float *denom, *nw, *slots;
 };
 
@@ -55,13 +55,13 @@ BackpropBufs carve(void* ws, int64_t n, int64_t num_bags) {
   p += pad(b.dedup_bytes);
   b.counts = p;
   p += pad(8 * un);
-  b.inverse = p;
-  p += pad(8 * un);
   b.doff = p;
   p += pad(8 * (un + 1));
   b.kidx = reinterpret_cast<uint32_t*>(p);
   p += pad(4 * un);
   b.rows = reinterpret_cast<uint32_t*>(p);
+  p += pad(4 * un);
+  b.by_key = reinterpret_cast<uint32_t*>(p);
   p += pad(4 * un);
   b.nw = reinterpret_cast<float*>(p);
   p += pad(4 * un);
@@ -77,7 +77,7 @@ BackpropBufs carve(void* ws, int64_t n, int64_t num_bags) {
 
 size_t backprop_workspace_bytes(int64_t n, int64_t num_bags, int64_t dim) {
   const size_t un = (size_t)std::max<int64_t>(n, 1);
-  return pad(dedup_workspace_bytes(n)) + 2 * pad(8 * un) + pad(8 * (un + 1)) + 3 * pad(4 * un) +
+  return pad(dedup_workspace_bytes(n)) + pad(8 * un) + pad(8 * (un + 1)) + 4 * pad(4 * un) +
          pad(4 * (size_t)std::max<int64_t>(num_bags, 1)) + pad(4 * (un / kPieceBlock + 2)) +
          slot_bytes(n, dim);
 }
@@ -123,10 +123,9 @@ int64_t pooling_backprop_run(int key_bytes, int64_t n, const void* keys, int poo
   if (mode == kBackpropMean || mode == kBackpropWMean)
     NVE_HIP(launch_bag_denom(csr, key_bytes, num_bags, hotness, weights, wdt, mode == kBackpropWMean,
                              b.denom, s));
-  const PositionGrad pg{mode, csr, key_bytes, num_bags, hotness, weights, wdt, b.denom, b.rows, b.nw};
-  const DedupHead* head_dev = nullptr;
-  dedup_run(key_bytes, n, keys, unique_out, b.counts, b.inverse, b.doff, b.dedup_ws, b.dedup_bytes, s,
-            b.kidx, &head_dev, exact, &pg);
+  const PositionGrad pg{mode, csr, key_bytes, num_bags, hotness, weights, wdt, b.denom, b.rows, b.nw, b.by_key};
+  dedup_run(key_bytes, n, keys, unique_out, b.counts, nullptr, b.doff, b.dedup_ws, b.dedup_bytes, s,
+            b.kidx, true, exact, &pg);
 
   // (3) pieces, then the keys that cross a block edge
   PieceArgs a{};
@@ -146,7 +145,7 @@ int64_t pooling_backprop_run(int key_bytes, int64_t n, const void* keys, int poo
   const int weighted = (mode == kBackpropWSum || mode == kBackpropMean || mode == kBackpropWMean) ? 1 : 0;
   NVE_HIP(launch_piece_pool(a, f16, weighted, s));
   NVE_HIP(launch_piece_combine(a, f16, s));
-  const DedupHead h = read_back(head_dev, s);
+  const DedupHead h = dedup_head(s);
   if (!exact && dedup_spec_failed(h))  // keys differ above the speculated sort bits: all again, exactly
     return pooling_backprop_run(key_bytes, n, keys, pooling, sparse, offsets, num_bags, hotness, weights, wdt,
                                 grads_in, gdt, dim, unique_out, grads_out, ws, ws_bytes, s, true);

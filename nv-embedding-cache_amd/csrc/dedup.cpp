@@ -4,6 +4,8 @@
 // 2^30 keys sort instead and gather in key order).
 #include "dedup.hpp"
 
+#include <algorithm>
+
 #include "kernels/backprop_launch.hpp"
 #include "kernels/cache_launch.hpp"
 #include "kernels/dedup_launch.hpp"
@@ -26,7 +28,8 @@ struct DedupBufs {
   DedupHead* head;
   uint64_t* span_part;
   uint64_t *ka, *kb;
-  uint32_t *va, *vb, *heads, *start;
+  uint32_t *va, *vb;
+  uint64_t* run_state;
   void* sort_tmp;
 };
 
@@ -47,10 +50,8 @@ DedupBufs carve(void* ws, int64_t n) {
   p += pad(4 * n);
   d.vb = reinterpret_cast<uint32_t*>(p);
   p += pad(4 * n);
-  d.heads = reinterpret_cast<uint32_t*>(p);
-  p += pad(4 * n);
-  d.start = reinterpret_cast<uint32_t*>(p);
-  p += pad(4 * (n + 1));
+  d.run_state = reinterpret_cast<uint64_t*>(p);
+  p += pad(8 * (size_t)run_state_words(n));
   d.sort_tmp = p;
   return d;
 }
@@ -68,66 +69,54 @@ constexpr int64_t kHashGatherMaxKeys = int64_t(1) << 30;
 
 size_t dedup_workspace_bytes(int64_t n) {
   if (n < 1) n = 1;
-  const size_t sort = 256 + pad(8 * (size_t)dedup_span_parts(n)) + 2 * pad(8 * n) + 4 * pad(4 * n) +
-                      pad(4 * (n + 1)) + radix_sort_temp_bytes(n);
+  const size_t sort = 256 + pad(8 * (size_t)dedup_span_parts(n)) + 2 * pad(8 * n) + 2 * pad(4 * n) +
+                      pad(8 * (size_t)run_state_words(n)) + radix_sort_temp_bytes(n);
   const size_t hash = n <= kHashGatherMaxKeys ? hash_gather_bytes(n) : 0;
   return sort > hash ? sort : hash;
 }
 
+DedupHead dedup_head(hipStream_t s) {
+  NVE_HIP(hipStreamSynchronize(s));
+  return *static_cast<DedupHead*>(pinned_slot());
+}
+
 int64_t dedup_run(int key_bytes, int64_t n, const void* keys, void* unique, void* counts,
                   void* inverse, void* offsets, void* ws, size_t ws_bytes, hipStream_t s,
-                  uint32_t* pos_key, const DedupHead** head_dev, bool exact, const PositionGrad* pg) {
+                  uint32_t* pos_key, bool later, bool exact, const PositionGrad* pg) {
   if (n <= 0) return 0;
   NVE_CHECK_ARG(n <= (int64_t)UINT32_MAX, "Too many keys for one dedup");
   NVE_CHECK_ARG(ws != nullptr && ws_bytes >= dedup_workspace_bytes(n), "Workspace too small");
   DedupBufs b = carve(ws, n);
-  // a single key needs no sort: it takes the exact path, which sorts nothing
-  if (n < 2) exact = true;
-  int alt = 0;
-  if (exact) {
-    NVE_HIP(launch_dedup_prep(keys, key_bytes, n, 1, b.ka, b.va, s));
-    NVE_HIP(launch_fill_u64(reinterpret_cast<uint64_t*>(&b.head->span), 1, 0, s));
-    NVE_HIP(key_span(b.ka, n, &b.head->span, s));
-    const int bits = bits_for(read_back(&b.head->span, s));
-    NVE_HIP(radix_sort_pairs(b.ka, b.va, b.kb, b.vb, n, 0, bits, b.sort_tmp, &alt, s));
+  const DedupOut out{key_bytes, unique,  counts,
+                     inverse,   offsets, pos_key,
+                     b.head,    static_cast<DedupHead*>(pinned_slot()), pg != nullptr ? *pg : PositionGrad{}};
+  if (n <= kSmallDedupKeys) {
+    NVE_HIP(launch_dedup_small(keys, n, out, s));
   } else {
-    // the first pass reads the caller's keys and writes each tile's span part;
-    // the outputs' workgroup 0 reduces them and whoever reads the head checks
-    const RadixSource src{keys, key_bytes, 1, b.span_part};
-    NVE_HIP(radix_sort_pairs(b.ka, b.va, b.kb, b.vb, n, 0, kSpecSortBits, b.sort_tmp, &alt, s, &src));
-  }
-  const uint64_t* ks = alt ? b.kb : b.ka;
-  const uint32_t* vs = alt ? b.vb : b.va;
-  if (run_blocks(n) <= kRunMaxBlocks) {
-    // every output in two launches (block scratch in the heads / start arrays)
-    NVE_HIP(launch_dedup_runs(ks, vs, n, key_bytes, unique, counts, inverse, offsets, pos_key, &b.head->total,
-                              b.heads, reinterpret_cast<int64_t*>(b.start), exact ? nullptr : b.span_part,
-                              exact ? nullptr : &b.head->span, pg, s));
-    if (head_dev != nullptr) {
-      *head_dev = b.head;
-      return -1;
+    int alt = 0;
+    const int64_t run_words = run_state_words(n);
+    if (exact) {
+      NVE_HIP(launch_dedup_prep(keys, key_bytes, n, 1, b.ka, b.va, s));
+      NVE_HIP(launch_fill_u64(reinterpret_cast<uint64_t*>(&b.head->span), 1, 0, s));
+      NVE_HIP(key_span(b.ka, n, &b.head->span, s));
+      // at least one pass (equal keys differ in no bit): it clears the run state
+      const int bits = std::max(1, bits_for(read_back(&b.head->span, s)));
+      NVE_HIP(radix_sort_pairs(b.ka, b.va, b.kb, b.vb, n, 0, bits, b.sort_tmp, &alt, s, nullptr, b.run_state,
+                               run_words, pg));
+    } else {
+      // the sort reads the caller's keys and writes span parts; the runs'
+      // first tile reduces them and whoever reads the head checks
+      const RadixSource src{keys, key_bytes, 1, b.span_part};
+      NVE_HIP(radix_sort_pairs(b.ka, b.va, b.kb, b.vb, n, 0, kSpecSortBits, b.sort_tmp, &alt, s, &src, b.run_state,
+                               run_words, pg));
     }
-    const DedupHead h = read_back(b.head, s);
-    if (!exact && dedup_spec_failed(h))
-      return dedup_run(key_bytes, n, keys, unique, counts, inverse, offsets, ws, ws_bytes, s, pos_key, nullptr,
-                       true, pg);
-    return (int64_t)h.total;
+    NVE_HIP(launch_dedup_runs(alt ? b.kb : b.ka, alt ? b.vb : b.va, n, exact ? nullptr : b.span_part, b.run_state,
+                              !exact && pg != nullptr && carries_rows(pg->mode), out, s));
   }
-  NVE_HIP(launch_run_heads(ks, n, b.heads, s));
-  NVE_HIP(exclusive_scan_u32(b.heads, n, &b.head->total, b.sort_tmp, s));
-  NVE_HIP(launch_dedup_outputs(ks, vs, b.heads, n, key_bytes, unique, inverse, offsets, b.start, pos_key,
-                               exact ? nullptr : b.span_part, exact ? nullptr : &b.head->span, s));
-  if (pg != nullptr) NVE_HIP(launch_backprop_prep(inverse, key_bytes, n, *pg, s));
-  if (head_dev != nullptr) {  // the caller reads the head when it needs it
-    NVE_HIP(launch_dedup_counts(b.start, (uint32_t)n, &b.head->total, key_bytes, counts, s));
-    *head_dev = b.head;
-    return -1;
-  }
-  const DedupHead h = read_back(b.head, s);
+  if (later) return -1;
+  const DedupHead h = dedup_head(s);
   if (!exact && dedup_spec_failed(h))
-    return dedup_run(key_bytes, n, keys, unique, counts, inverse, offsets, ws, ws_bytes, s, pos_key, nullptr,
-                     true, pg);
-  NVE_HIP(launch_dedup_counts(b.start, h.total, nullptr, key_bytes, counts, s));
+    return dedup_run(key_bytes, n, keys, unique, counts, inverse, offsets, ws, ws_bytes, s, pos_key, false, true, pg);
   return (int64_t)h.total;
 }
 

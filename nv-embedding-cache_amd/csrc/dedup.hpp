@@ -6,19 +6,11 @@
 
 #include <cstddef>
 
-#include "kernels/backprop_launch.hpp"
+#include "kernels/dedup_launch.hpp"
 
 namespace nve_amd {
 
 size_t dedup_workspace_bytes(int64_t n);
-
-// The unique count and the key span of a dedup, side by side at the start of
-// its workspace so that one readback fetches both.
-struct DedupHead {
-  uint32_t total;           // unique keys
-  uint32_t pad;
-  unsigned long long span;  // OR over the keys of key ^ key[0] (sort keys): the bits where they differ
-};
 
 // The sort first assumes that the keys differ only below this bit (rows of
 // tables up to 2^27: three 9-bit passes) and learns whether they did from the
@@ -31,18 +23,19 @@ inline bool dedup_spec_failed(const DedupHead& h) { return (h.span >> kSpecSortB
 // Sorted unique keys, counts, stable inverse map and exclusive offsets (all of
 // the key type); returns the number of unique keys (synchronizes the stream).
 // pos_key (optional, n entries): the unique index of each position of the
-// dedup order.  head_dev (optional): instead of reading the head back (a
-// stream synchronization), return -1 and point *head_dev at the head in the
-// workspace (valid once the stream reaches it, until the workspace is
-// reused); the caller reads it and, if dedup_spec_failed, runs again with
-// exact = true.  exact: read the key span back first and sort on exactly its
-// bits (never needs a second run).
+// dedup order.  later: instead of waiting for the head (a stream
+// synchronization), return -1; the caller calls dedup_head once it has queued
+// what follows (from the same thread, before another dedup) and, if
+// dedup_spec_failed, runs again with exact = true.  exact: read the key span
+// back first and sort on exactly its bits (never needs a second run).
 // pg (optional): also each dedup position's gradient row and weight (the
 // backprop's per-position step, done on the way).
 int64_t dedup_run(int key_bytes, int64_t n, const void* keys, void* unique, void* counts,
                   void* inverse, void* offsets, void* ws, size_t ws_bytes, hipStream_t s,
-                  uint32_t* pos_key = nullptr, const DedupHead** head_dev = nullptr, bool exact = false,
+                  uint32_t* pos_key = nullptr, bool later = false, bool exact = false,
                   const PositionGrad* pg = nullptr);
+// The head of this thread's last dedup_run on stream s (synchronizes it).
+DedupHead dedup_head(hipStream_t s);
 
 // out[i] = table row keys[i] for keys in [0, num_rows), each distinct row read
 // from the table once (asynchronous).

@@ -1,6 +1,5 @@
 // backprop.hip -- kernels of the training backprop (the sparse gradient of a
-// lookup): bag denominators, the gradient row and weight of every key
-// position in dedup order, and the two summation kernels.
+// lookup): bag denominators and the two summation kernels.
 //
 // Summation order (fixed, and the CPU oracle's): the dedup order of the
 // positions is cut into blocks of kPieceBlock; a piece is one key's positions
@@ -22,7 +21,6 @@
 #include "backprop_launch.hpp"
 #include "device_common.cuh"
 #include "lane_moves.cuh"
-#include "position_grad.cuh"
 
 namespace nve_amd {
 
@@ -56,13 +54,6 @@ __global__ __launch_bounds__(256) void bag_denom_kernel(const void* offsets, int
   float acc = 0.0f;
   for (int64_t p = s; p < e; ++p) acc += load_weight(weights, wdt, p);
   denom[b] = acc;
-}
-
-// rows / nw of dedup position j (key position p = inverse[j])
-__global__ __launch_bounds__(256) void backprop_prep_kernel(const void* inverse, int key_bytes, int64_t n,
-                                                            PositionGrad g) {
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < n) position_grad(g, j, load_key(inverse, key_bytes, j));
 }
 
 constexpr int kPieceThreads = 256;
@@ -351,14 +342,6 @@ hipError_t launch_bag_denom(const void* offsets, int key_bytes, int64_t num_bags
   if (num_bags <= 0) return hipSuccess;
   hipLaunchKernelGGL(bag_denom_kernel, dim3((unsigned)((num_bags + 255) / 256)), dim3(256), 0, stream,
                      offsets, key_bytes, num_bags, hotness, weights, wdt, wmean, denom);
-  return hipGetLastError();
-}
-
-hipError_t launch_backprop_prep(const void* inverse, int key_bytes, int64_t n, const PositionGrad& g,
-                                hipStream_t stream) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(backprop_prep_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
-                     inverse, key_bytes, n, g);
   return hipGetLastError();
 }
 

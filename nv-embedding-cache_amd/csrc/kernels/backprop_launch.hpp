@@ -25,6 +25,7 @@ constexpr int kLightPieces = 32;   // a crossing key of more pieces is added by 
 // What the backprop needs per key position: how its gradient row and weight
 // follow from its position (the bags, weights and bag denominators), and
 // where they go (rows / nw, one entry per dedup position; rows null: none).
+// by_key: scratch, the gradient row of each key position (pooled modes).
 struct PositionGrad {
   int mode;             // kBackprop*
   const void* offsets;  // CSR offsets of the key type, or null (Fixed hotness)
@@ -36,11 +37,8 @@ struct PositionGrad {
   const float* denom;   // Mean / WeightedMean: per bag
   uint32_t* rows;
   float* nw;
+  uint32_t* by_key;
 };
-
-// rows / nw of every dedup position j from inverse[j] (its key position).
-hipError_t launch_backprop_prep(const void* inverse, int key_bytes, int64_t n, const PositionGrad& g,
-                                hipStream_t stream);
 
 struct PieceArgs {
   const uint32_t* kidx;  // unique index of each dedup position

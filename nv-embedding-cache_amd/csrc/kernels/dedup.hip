@@ -3,11 +3,10 @@
 //
 // dedup: stable radix sort of (key, position) -> runs of equal keys -> per
 // run: unique key, start offset, count; per position: inverse = original
-// position in key order.  The runs take two launches (per-block head counts,
-// then every output with the blocks before as carry-in) up to kRunMaxBlocks
-// blocks, else run heads -> exclusive scan -> outputs -> counts.  Outputs
-// match the reference's: unique keys ascending (signed order), counts, the
-// stable inverse map and exclusive offsets.
+// position in key order.  The runs take one launch; a batch of at most
+// kSmallDedupKeys keys is sorted and written by one workgroup in one launch.
+// Outputs match the reference's: unique keys ascending (signed order), counts,
+// the stable inverse map and exclusive offsets.
 //
 // dedup-then-gather needs no order, so it dedups by hashing instead of
 // sorting (three launches instead of eleven): every distinct key of a
@@ -19,19 +18,25 @@
 // position copies its owner's output row (UnpackDedup, cuda_utils.cuh:24-79).
 #include "device_common.cuh"
 #include "dedup_launch.hpp"
+#include "lane_moves.cuh"
 #include "position_grad.cuh"
 #include "sort_launch.hpp"
+#include "tile_rank.cuh"
 
 namespace nve_amd {
 
-// OR of x over the 256 threads of the workgroup, in every thread (all threads call it)
+// OR of x over the NT threads of the workgroup, in every thread (all threads call it)
+template <int NT>
 __device__ __forceinline__ uint64_t block_or(uint64_t x) {
-  __shared__ uint64_t red[4];
+  __shared__ uint64_t red[NT / 64];
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) x |= __shfl_xor(x, o);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
   __syncthreads();
-  return red[0] | red[1] | red[2] | red[3];
+  uint64_t all = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) all |= red[w];
+  return all;
 }
 
 __global__ __launch_bounds__(256) void dedup_prep_kernel(const void* keys, int key_bytes, int64_t n,
@@ -44,228 +49,323 @@ __global__ __launch_bounds__(256) void dedup_prep_kernel(const void* keys, int k
   }
 }
 
-// inverse[i] = position of the i-th key in key order; at a run head:
-// unique[u] = key, offsets[u] = i (= start[u]); start[U] = n.
-// span_part (optional, nparts words): workgroup 0 also ORs the prep's span
-// parts into *span_out.
-__global__ __launch_bounds__(256) void dedup_outputs_kernel(const uint64_t* ks, const uint32_t* vs,
-                                                            const uint32_t* scan, int64_t n,
-                                                            int key_bytes, void* unique,
-                                                            void* inverse, void* offsets,
-                                                            uint32_t* start, uint32_t* pos_key,
-                                                            const uint64_t* span_part, int64_t nparts,
-                                                            unsigned long long* span_out) {
-  if (span_part != nullptr && blockIdx.x == 0) {  // uniform over the workgroup
-    uint64_t a = 0;
-    for (int64_t j = threadIdx.x; j < nparts; j += blockDim.x) a |= span_part[j];
-    a = block_or(a);
-    if (threadIdx.x == 0) *span_out = a;
-  }
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  store_key(inverse, key_bytes, i, (int64_t)vs[i]);
-  const bool head = (i == 0 || ks[i] != ks[i - 1]);
-  if (pos_key != nullptr) pos_key[i] = head ? scan[i] : scan[i] - 1u;  // unique index of position i
-  if (head) {
-    const uint32_t u = scan[i];
-    store_key(unique, key_bytes, u, unflip_key(ks[i], key_bytes));
-    store_key(offsets, key_bytes, u, i);
-    start[u] = (uint32_t)i;
-  }
-  if (i == n - 1) start[scan[i] + (head ? 1u : 0u)] = (uint32_t)n;
-}
-
-// u_dev (optional): the unique count in device memory, for a grid sized by an
-// upper bound without reading the count back first.
-__global__ __launch_bounds__(256) void dedup_counts_kernel(const uint32_t* start, uint32_t u_n,
-                                                           const uint32_t* u_dev, int key_bytes,
-                                                           void* counts) {
-  const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t m = u_dev != nullptr ? *u_dev : u_n;
-  if (u < m) store_key(counts, key_bytes, u, (int64_t)(start[u + 1] - start[u]));
-}
-
 // ---------------------------------------------------------------------------
-// runs of the sorted keys in two launches (batches of up to kRunMaxBlocks
-// blocks of kRunBlock keys): run_block_kernel counts each block's run heads
-// and notes its last head; run_outputs_kernel takes the sums and maxima of
-// the blocks before its own as carry-in (so no scan launch sits between), and
-// writes every output of the dedup: per position its inverse entry and unique
-// index, per run its key and offset at the head and its count at the tail.
+// runs of the sorted keys, every output of the dedup in one launch: per position
+// its inverse entry and unique index, per run its key and offset at the head
+// and its count at the tail.  A 1024-thread workgroup per 4096 positions counts
+// its run heads, publishes the count and its last head, and takes those of the
+// tiles before by walking back over them, while the other waves already write
+// their positions' gradient rows.  Bound: the latency of that chain, and the
+// tile counter (one address: with 1024-key tiles 256 increments queued, 12.5 us
+// for 262,144 keys, 9.7 with 4096).  Counting heads in a launch of its own and
+// finding each position's bag here took 17.9 us.
 // ---------------------------------------------------------------------------
-constexpr int kRunThreads = 256;
+constexpr int kRunThreads = 1024;
 constexpr int kRunItems = 4;
 constexpr int kRunBlock = kRunThreads * kRunItems;
 
-// Block-wide exclusive sum of c and exclusive maximum of l over thread order
-// (every thread calls it); *sum = the block's total of c.
-__device__ __forceinline__ void block_scan_sum_max(uint32_t c, int64_t l, uint32_t* ex_c, int64_t* ex_l,
-                                                   uint32_t* sum) {
-  __shared__ uint32_t wc[kRunThreads / 64];
-  __shared__ int64_t wl[kRunThreads / 64];
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  uint32_t ic = c;  // inclusive within the wave
-  int64_t il = l;
+// The runs of a workgroup's NT * ITEMS positions, position base + j * NT + tid
+// in round j of thread tid, so that every load and store is of consecutive
+// positions.  A wave's 64 positions of a round are a segment: its run heads
+// are a ballot, its place the scan of the segments' head counts.
+template <int NT, int ITEMS>
+struct RunTile {
+  static constexpr int kWaves = NT / 64;
+  static constexpr int kSegs = ITEMS * kWaves;
+  static_assert(kSegs <= 64, "one wave scans the segments");
+  uint32_t seg_c[kSegs];  // heads of the tile before the segment
+  int seg_l[kSegs];       // last head of the tile before it (-1: none)
+  uint32_t sum;           // heads of the tile
+  int max;                // its last head (-1: none)
+};
+
+// heads[j] = the wave's run heads of round j; t: filled for the whole
+// workgroup (every thread calls it; key_at(i) is read for i in [0, n)).
+template <int NT, int ITEMS, typename K>
+__device__ __forceinline__ void find_runs(RunTile<NT, ITEMS>& t, const K& key_at, int64_t base, int64_t n,
+                                          uint64_t (&heads)[ITEMS]) {
+  constexpr int kSegs = RunTile<NT, ITEMS>::kSegs;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t pc = __shfl_up(ic, o);
-    const int64_t pl = __shfl_up(il, o);
-    if (lane >= o) {
-      ic += pc;
-      il = pl > il ? pl : il;
+  for (int j = 0; j < ITEMS; ++j) {
+    const int64_t i = base + j * NT + tid;
+    heads[j] = __ballot(i < n && (i == 0 || key_at(i) != key_at(i - 1)));
+    const int seg = j * (NT / 64) + wave;
+    if (lane == 0) {
+      t.seg_c[seg] = (uint32_t)__popcll(heads[j]);
+      t.seg_l[seg] = heads[j] ? j * NT + wave * 64 + 63 - __builtin_clzll(heads[j]) : -1;
     }
   }
-  if (lane == 63) {
-    wc[wave] = ic;
-    wl[wave] = il;
-  }
   __syncthreads();
-  uint32_t bc = 0;
-  int64_t bl = -1;
-  for (int w = 0; w < wave; ++w) {
-    bc += wc[w];
-    bl = wl[w] > bl ? wl[w] : bl;
-  }
-  uint32_t tot = 0;
-  for (int w = 0; w < kRunThreads / 64; ++w) tot += wc[w];
-  // exclusive: inclusive minus own, maximum of the lanes before
-  const int64_t prev_l = __shfl_up(il, 1);
-  *ex_c = bc + ic - c;
-  const int64_t lane_l = lane > 0 ? prev_l : -1;
-  *ex_l = lane_l > bl ? lane_l : bl;
-  *sum = tot;
-}
-
-// blk_count[b] = run heads in block b, blk_last[b] = its last head position (-1: none)
-__global__ __launch_bounds__(kRunThreads) void run_block_kernel(const uint64_t* ks, int64_t n,
-                                                                uint32_t* blk_count, int64_t* blk_last) {
-  const int64_t base = (int64_t)blockIdx.x * kRunBlock;
-  uint32_t c = 0;
-  int64_t l = -1;
-#pragma unroll 4
-  for (int j = 0; j < kRunItems; ++j) {
-    const int64_t i = base + (int64_t)j * kRunThreads + threadIdx.x;  // coalesced
-    if (i < n && (i == 0 || ks[i] != ks[i - 1])) {
-      ++c;
-      l = i;
+  if (tid < 64) {
+    const uint32_t c = tid < kSegs ? t.seg_c[tid] : 0u;
+    int l = tid < kSegs ? t.seg_l[tid] : -1;
+    const uint32_t inc = wave_sum_scan(c);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int p = __shfl_up(l, o);
+      if (lane >= o) l = p > l ? p : l;
+    }
+    const int before = __shfl_up(l, 1);
+    if (tid < kSegs) {
+      t.seg_c[tid] = inc - c;
+      t.seg_l[tid] = lane > 0 ? before : -1;
+    }
+    if (tid == 63) {
+      t.sum = inc;
+      t.max = l;
     }
   }
-  uint32_t ex_c, sum;
-  int64_t ex_l;
-  block_scan_sum_max(c, l, &ex_c, &ex_l, &sum);
-  // the block's last head: the maximum over all threads
-  __shared__ int64_t last;
-  if (threadIdx.x == kRunThreads - 1) last = l > ex_l ? l : ex_l;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    blk_count[blockIdx.x] = sum;
-    blk_last[blockIdx.x] = last;
+}
+
+// The outputs of the tile: u0 heads before it, h0 the last of them.
+template <int NT, int ITEMS, typename K>
+__device__ __forceinline__ void emit_runs(const RunTile<NT, ITEMS>& t, const K& key_at, const DedupOut& o,
+                                          const uint64_t (&heads)[ITEMS], const uint32_t (&pos)[ITEMS], int64_t base,
+                                          int64_t n, uint32_t u0, int64_t h0) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint64_t upto = ~0ull >> (63 - lane);
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    const int64_t i = base + j * NT + tid;
+    if (i >= n) continue;
+    const int seg = j * (NT / 64) + wave;
+    const uint64_t m = heads[j] & upto;
+    const uint32_t u = u0 + t.seg_c[seg] + (uint32_t)__popcll(m) - 1u;
+    const uint64_t key = key_at(i);
+    if ((heads[j] >> lane) & 1u) {
+      store_key(o.unique, o.key_bytes, u, unflip_key(key, o.key_bytes));
+      store_key(o.offsets, o.key_bytes, u, i);
+    }
+    if (o.inverse != nullptr) store_key(o.inverse, o.key_bytes, i, (int64_t)pos[j]);
+    if (o.pos_key != nullptr) o.pos_key[i] = u;
+    if (i == n - 1 || key != key_at(i + 1)) {  // the run ends here
+      const int64_t start = m ? base + j * NT + wave * 64 + 63 - __builtin_clzll(m)
+                              : (t.seg_l[seg] >= 0 ? base + t.seg_l[seg] : h0);
+      store_key(o.counts, o.key_bytes, u, i + 1 - start);
+    }
   }
 }
 
-struct RunOutputs {
+// The unique count and the keys' span to the head in device memory and, where
+// given, to its copy in pinned host memory.
+__device__ __forceinline__ void write_total(const DedupOut& o, uint32_t total) {
+  o.head->total = total;
+  if (o.host_head != nullptr) o.host_head->total = total;
+}
+__device__ __forceinline__ void write_span(const DedupOut& o, unsigned long long span) {
+  o.head->span = span;
+  if (o.host_head != nullptr) o.host_head->span = span;
+}
+
+struct RunArgs {
   const uint64_t* ks;
   const uint32_t* vs;
   int64_t n;
-  const uint32_t* blk_count;
-  const int64_t* blk_last;
-  int key_bytes;
-  void* unique;
-  void* counts;
-  void* inverse;
-  void* offsets;
-  uint32_t* pos_key;   // optional
-  uint32_t* total;     // the unique count, written by the last block
-  const uint64_t* span_part;  // optional: block 0 ORs these into *span_out
+  const uint64_t* span_part;  // null: no span to check
   int64_t nparts;
-  unsigned long long* span_out;
-  PositionGrad pg;            // pg.rows non-null: each position's gradient row and weight too
+  uint64_t* state;  // tile counter, then per tile its head count and its last head + 1
+  bool carried;     // vs holds gradient rows
+  DedupOut out;
 };
 
-__global__ __launch_bounds__(kRunThreads) void run_outputs_kernel(RunOutputs a) {
-  if (a.span_part != nullptr && blockIdx.x == 0) {  // uniform over the workgroup
+__global__ __launch_bounds__(kRunThreads) void run_outputs_kernel(RunArgs a) {
+  __shared__ uint32_t s_tile, s_u0;
+  __shared__ int64_t s_h0;
+  const int tid = threadIdx.x;
+  if (tid == 0) s_tile = take_tile(a.state);
+  __syncthreads();
+  const int64_t tile = s_tile;
+  if (tile == 0) {  // uniform over the workgroup
     uint64_t x = 0;
-    for (int64_t j = threadIdx.x; j < a.nparts; j += blockDim.x) x |= a.span_part[j];
-    x = block_or(x);
-    if (threadIdx.x == 0) *a.span_out = x;
+    if (a.span_part != nullptr)
+      for (int64_t j = tid; j < a.nparts; j += kRunThreads) x |= a.span_part[j];
+    x = block_or<kRunThreads>(x);
+    if (tid == 0) write_span(a.out, x);
   }
-  // carry-in: heads before this block, and the last head before it
-  uint32_t u0;
-  int64_t h0;
-  {
-    __shared__ uint32_t in_c[kRunThreads / 64];
-    __shared__ int64_t in_l[kRunThreads / 64];
-    uint32_t c = 0;
-    int64_t l = -1;
-    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += blockDim.x) {
-      c += a.blk_count[b];
-      l = a.blk_last[b] > l ? a.blk_last[b] : l;
-    }
+  const int64_t base = tile * kRunBlock;
+  const auto key_at = [&](int64_t i) { return a.ks[i]; };
+  uint32_t pos[kRunItems];
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      c += __shfl_xor(c, o);
-      const int64_t p = __shfl_xor(l, o);
-      l = p > l ? p : l;
+  for (int j = 0; j < kRunItems; ++j) {
+    const int64_t i = base + j * kRunThreads + tid;
+    pos[j] = i < a.n ? a.vs[i] : 0;
+  }
+  __shared__ RunTile<kRunThreads, kRunItems> runs;
+  uint64_t run_heads[kRunItems];
+  find_runs<kRunThreads, kRunItems>(runs, key_at, base, a.n, run_heads);
+  const uint32_t sum = runs.sum;
+  const uint64_t max1 = runs.max >= 0 ? (uint64_t)(base + runs.max + 1) : 0;  // last head + 1, 0: none
+  if (tid < 64) {
+    // publish, then the tiles before: the sum of their head counts and the
+    // nearest one's last head, 64 of them at a time.  Every one of them has
+    // started and publishes without waiting for another, so each wait ends.
+    uint64_t* const word = a.state + 1 + 2 * tile;
+    if (tid < 2) store_state(word + tid, (tile == 0 ? kStateBefore : kStateOwn) | (tid == 0 ? sum : max1));
+    uint64_t heads = 0, last = 0;  // last head + 1, 0: none
+    bool open_c = tile > 0, open_l = tile > 0;  // uniform over the wave
+    for (int64_t top = tile - 1; top >= 0 && (open_c || open_l); top -= 64) {
+      const int64_t t = top - tid;
+      uint64_t wc = kStateBefore, wl = kStateBefore;  // before the first tile: nothing
+      if (t >= 0) {
+        do {
+          wc = load_state(a.state + 1 + 2 * t);
+          wl = load_state(a.state + 2 + 2 * t);
+        } while (wc < kStateOwn || wl < kStateOwn);
+      }
+      if (open_c) {
+        const uint64_t closed = __ballot(wc >= kStateBefore);
+        const int end = closed ? __builtin_ctzll(closed) : 63;  // the last lane to add
+        uint32_t v = tid <= end ? (uint32_t)(wc & kStateCount) : 0u;  // heads fit 32 bits
+        v = wave_sum_scan(v);
+        heads += (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+        open_c = closed == 0;
+      }
+      if (open_l) {
+        const uint64_t known = __ballot(wl >= kStateBefore || (wl & kStateCount) != 0);
+        if (known) {
+          last = __shfl(wl, __builtin_ctzll(known)) & kStateCount;
+          open_l = false;
+        }
+      }
     }
-    if ((threadIdx.x & 63) == 0) {
-      in_c[threadIdx.x >> 6] = c;
-      in_l[threadIdx.x >> 6] = l;
+    if (tid == 0) {
+      s_u0 = (uint32_t)heads;
+      s_h0 = (int64_t)last - 1;
+      if (tile > 0) {
+        store_state(word, kStateBefore | (heads + sum));
+        store_state(word + 1, kStateBefore | (max1 ? max1 : last));
+      }
+      if (tile == gridDim.x - 1) write_total(a.out, (uint32_t)heads + sum);
+    }
+  }
+  if (a.out.pg.rows != nullptr) {
+    const auto row_at = [&](uint32_t p) { return a.out.pg.by_key[p]; };
+    position_grads<kRunItems>(a.out.pg, a.carried, row_at, base + tid, kRunThreads, a.n, pos);
+  }
+  __syncthreads();
+  emit_runs<kRunThreads, kRunItems>(runs, key_at, a.out, run_heads, pos, base, a.n, s_u0, s_h0);
+}
+
+// ---------------------------------------------------------------------------
+// The whole dedup of a small batch (at most 1024 * ITEMS keys) in one workgroup
+// and one launch: the keys stay in LDS between the passes, and the passes cover
+// exactly the bits in which the keys differ, so nothing is assumed about them.
+// Bound: the latency of one workgroup's passes; the sort and the runs took six
+// launches (dedup of 500 keys 58.8 -> 19.0 us, 2,000 keys 58.2 -> 25.7, 4,096 keys 59.3 ->
+// 28.3; one workgroup of 8,192 keys took as long as the radix sort, 50 us).
+// ---------------------------------------------------------------------------
+template <int ITEMS>
+__global__ __launch_bounds__(1024) void dedup_small_kernel(const void* keys, int n, DedupOut o) {
+  constexpr int RB = 9;  // as the radix sort: three passes for the keys of tables of up to 2^27 rows
+  constexpr int kBins = 1 << RB;
+  constexpr int kWaves = 16;
+  __shared__ uint64_t sk[1024 * ITEMS];
+  __shared__ uint32_t sv[1024 * ITEMS];
+  __shared__ uint32_t rows[1024 * ITEMS];
+  __shared__ uint32_t cnt[kWaves][kBins];
+  __shared__ uint32_t lstart[kBins];
+  __shared__ uint32_t wsum[kBins / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int li0 = wave * (64 * ITEMS) + lane;  // key r of the lane: li0 + 64 * r
+  uint64_t k[ITEMS];
+  uint32_t v[ITEMS];
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const int li = li0 + 64 * r;
+    k[r] = flip_key(load_key(keys, o.key_bytes, li < n ? li : 0), o.key_bytes);
+    v[r] = (uint32_t)li;
+  }
+  // pooled gradients: the row of every key position; values: rows where they do
+  const bool pooled = o.pg.rows != nullptr && o.pg.mode != kBackpropConcat;  // uniform
+  const bool carried = pooled && weight_from_row(o.pg.mode);
+  if (pooled) {
+    tile_rows<1024, 1024 * ITEMS>(o.pg, 0, rows);
+    if (carried) {
+#pragma unroll
+      for (int r = 0; r < ITEMS; ++r) v[r] = rows[li0 + 64 * r];
+    }
+  }
+  // the bits in which the keys differ (a lane past the end holds key 0)
+  uint64_t diff = 0;
+  const uint64_t k0 = flip_key(load_key(keys, o.key_bytes, 0), o.key_bytes);
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) diff |= k[r] ^ k0;
+  const uint64_t span = block_or<1024>(diff);
+  const int bits = span ? 64 - __builtin_clzll(span) : 0;
+
+  int shift = 0;
+  do {  // at least once, which lays the keys out in LDS
+    for (int d = tid; d < kWaves * kBins; d += 1024) (&cnt[0][0])[d] = 0;
+    __syncthreads();
+    uint32_t rank[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r)
+      rank[r] = wave_digit_rank<RB>((uint32_t)(k[r] >> shift) & (kBins - 1), li0 + 64 * r < n, cnt[wave]);
+    __syncthreads();
+    uint32_t own = 0, inc = 0;
+    if (tid < kBins) {
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        const uint32_t c = cnt[w][tid];
+        cnt[w][tid] = own;
+        own += c;
+      }
+      inc = wave_sum_scan(own);
+      if (lane == 63) wsum[wave] = inc;
     }
     __syncthreads();
-    u0 = 0;
-    h0 = -1;
+    if (tid < kBins) {
+      uint32_t ex = inc - own;
 #pragma unroll
-    for (int w = 0; w < kRunThreads / 64; ++w) {
-      u0 += in_c[w];
-      h0 = in_l[w] > h0 ? in_l[w] : h0;
+      for (int w = 0; w < kBins / 64; ++w)
+        if (w < wave) ex += wsum[w];
+      lstart[tid] = ex;
     }
-  }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+      if (li0 + 64 * r < n) {
+        const uint32_t d = (uint32_t)(k[r] >> shift) & (kBins - 1);
+        const uint32_t at = lstart[d] + cnt[wave][d] + rank[r];
+        sk[at] = k[r];
+        sv[at] = v[r];
+      }
+    }
+    __syncthreads();
+    shift += RB;
+    if (shift < bits) {
+#pragma unroll
+      for (int r = 0; r < ITEMS; ++r) {
+        const int li = li0 + 64 * r;
+        if (li < n) {
+          k[r] = sk[li];
+          v[r] = sv[li];
+        }
+      }
+    }
+  } while (shift < bits);
 
-  // this thread's kRunItems consecutive positions
-  const int64_t first = (int64_t)blockIdx.x * kRunBlock + (int64_t)threadIdx.x * kRunItems;
-  uint64_t k[kRunItems];
+  const auto key_at = [&](int64_t i) { return sk[i]; };
+  uint32_t pos[ITEMS];
 #pragma unroll
-  for (int j = 0; j < kRunItems; ++j) k[j] = first + j < a.n ? a.ks[first + j] : 0;
-  const uint64_t before = first > 0 && first - 1 < a.n ? a.ks[first - 1] : 0;
-  const uint64_t after = first + kRunItems < a.n ? a.ks[first + kRunItems] : 0;
-  uint32_t c = 0;
-  int64_t l = -1;
-#pragma unroll
-  for (int j = 0; j < kRunItems; ++j) {
-    const int64_t i = first + j;
-    const bool head = i < a.n && (i == 0 || k[j] != (j ? k[j - 1] : before));
-    if (head) {
-      ++c;
-      l = i;
-    }
+  for (int j = 0; j < ITEMS; ++j) {
+    const int i = j * 1024 + tid;
+    pos[j] = i < n ? sv[i] : 0;
   }
-  uint32_t ex_c, sum;
-  int64_t ex_l;
-  block_scan_sum_max(c, l, &ex_c, &ex_l, &sum);
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *a.total = u0 + sum;
-
-  // the run in progress at this thread's first position
-  uint32_t u = u0 + ex_c - 1u;  // wraps for position 0, which is a head
-  int64_t start = ex_l > h0 ? ex_l : h0;
-#pragma unroll
-  for (int j = 0; j < kRunItems; ++j) {
-    const int64_t i = first + j;
-    if (i >= a.n) break;
-    const bool head = i == 0 || k[j] != (j ? k[j - 1] : before);
-    if (head) {
-      ++u;
-      start = i;
-      store_key(a.unique, a.key_bytes, u, unflip_key(k[j], a.key_bytes));
-      store_key(a.offsets, a.key_bytes, u, i);
-    }
-    const uint32_t pos = a.vs[i];
-    store_key(a.inverse, a.key_bytes, i, (int64_t)pos);
-    if (a.pos_key != nullptr) a.pos_key[i] = u;
-    if (a.pg.rows != nullptr) position_grad(a.pg, i, (int64_t)pos);
-    const bool tail = i == a.n - 1 || k[j] != (j + 1 < kRunItems ? k[j + 1] : after);
-    if (tail) store_key(a.counts, a.key_bytes, u, i + 1 - start);
+  __shared__ RunTile<1024, ITEMS> runs;
+  uint64_t run_heads[ITEMS];
+  find_runs<1024, ITEMS>(runs, key_at, 0, n, run_heads);
+  if (tid == 0) {
+    write_total(o, runs.sum);
+    write_span(o, 0);
   }
+  if (o.pg.rows != nullptr) {
+    const auto row_at = [&](uint32_t p) { return rows[p]; };
+    position_grads<ITEMS>(o.pg, carried, row_at, tid, 1024, n, pos);
+  }
+  emit_runs<1024, ITEMS>(runs, key_at, o, run_heads, pos, 0, n, 0u, -1);
 }
 
 // ---------------------------------------------------------------------------
@@ -601,6 +701,8 @@ hipError_t launch_hash_dedup_gather(const void* keys, int key_bytes, int64_t n, 
 
 int64_t dedup_span_parts(int64_t n) { return radix_span_parts(n); }
 
+bool carries_rows(int mode) { return mode != kBackpropConcat && weight_from_row(mode); }
+
 hipError_t launch_dedup_prep(const void* keys, int key_bytes, int64_t n, int flip, uint64_t* k64,
                              uint32_t* v, hipStream_t stream) {
   if (n <= 0) return hipSuccess;
@@ -609,39 +711,24 @@ hipError_t launch_dedup_prep(const void* keys, int key_bytes, int64_t n, int fli
   return hipGetLastError();
 }
 
-hipError_t launch_dedup_outputs(const uint64_t* ks, const uint32_t* vs, const uint32_t* scan,
-                                int64_t n, int key_bytes, void* unique, void* inverse,
-                                void* offsets, uint32_t* start, uint32_t* pos_key,
-                                const uint64_t* span_part, unsigned long long* span_out,
-                                hipStream_t stream) {
+int64_t run_state_words(int64_t n) { return 1 + 2 * ((n + kRunBlock - 1) / kRunBlock); }
+
+hipError_t launch_dedup_runs(const uint64_t* ks, const uint32_t* vs, int64_t n, const uint64_t* span_part,
+                             uint64_t* state, bool carried, const DedupOut& out, hipStream_t stream) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(dedup_outputs_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, ks, vs, scan,
-                     n, key_bytes, unique, inverse, offsets, start, pos_key, span_part,
-                     dedup_span_parts(n), span_out);
+  const RunArgs a{ks, vs, n, span_part, dedup_span_parts(n), state, carried, out};
+  hipLaunchKernelGGL(run_outputs_kernel, dim3((unsigned)((n + kRunBlock - 1) / kRunBlock)), dim3(kRunThreads), 0,
+                     stream, a);
   return hipGetLastError();
 }
 
-int64_t run_blocks(int64_t n) { return (n + kRunBlock - 1) / kRunBlock; }
-
-hipError_t launch_dedup_runs(const uint64_t* ks, const uint32_t* vs, int64_t n, int key_bytes, void* unique,
-                             void* counts, void* inverse, void* offsets, uint32_t* pos_key, uint32_t* total,
-                             uint32_t* blk_count, int64_t* blk_last, const uint64_t* span_part,
-                             unsigned long long* span_out, const PositionGrad* pg, hipStream_t stream) {
+hipError_t launch_dedup_small(const void* keys, int64_t n, const DedupOut& out, hipStream_t stream) {
   if (n <= 0) return hipSuccess;
-  const int64_t nb = run_blocks(n);
-  if (nb > kRunMaxBlocks) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(run_block_kernel, dim3(nb), dim3(kRunThreads), 0, stream, ks, n, blk_count, blk_last);
-  RunOutputs a{ks, vs, n, blk_count, blk_last, key_bytes, unique, counts, inverse, offsets, pos_key, total,
-               span_part, dedup_span_parts(n), span_out, pg != nullptr ? *pg : PositionGrad{}};
-  hipLaunchKernelGGL(run_outputs_kernel, dim3(nb), dim3(kRunThreads), 0, stream, a);
-  return hipGetLastError();
-}
-
-hipError_t launch_dedup_counts(const uint32_t* start, uint32_t u_n, const uint32_t* u_dev,
-                               int key_bytes, void* counts, hipStream_t stream) {
-  if (u_n == 0) return hipSuccess;
-  hipLaunchKernelGGL(dedup_counts_kernel, dim3((u_n + 255) / 256), dim3(256), 0, stream, start, u_n,
-                     u_dev, key_bytes, counts);
+  if (n > kSmallDedupKeys) return hipErrorInvalidValue;
+  if (n <= 1024)
+    hipLaunchKernelGGL(dedup_small_kernel<1>, dim3(1), dim3(1024), 0, stream, keys, (int)n, out);
+  else
+    hipLaunchKernelGGL(dedup_small_kernel<4>, dim3(1), dim3(1024), 0, stream, keys, (int)n, out);
   return hipGetLastError();
 }
 

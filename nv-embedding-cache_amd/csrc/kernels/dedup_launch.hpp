@@ -8,35 +8,47 @@
 
 namespace nve_amd {
 
-// Words of the key-span parts the radix sort's first pass writes for n keys
-// (one per tile, radix_span_parts(n)).
+// The unique count and the key span of a dedup, side by side.
+struct DedupHead {
+  uint32_t total;           // unique keys
+  uint32_t pad;
+  unsigned long long span;  // OR over the keys of key ^ key[0] (sort keys): the bits where they differ
+};
+
+// Where a dedup's outputs go: unique keys, counts, inverse (optional) and offsets
+// of the key type, pos_key (optional) the unique index of every dedup position, the head
+// (and a copy in pinned host memory, optional); with pg.rows, each dedup
+// position's gradient row and weight.
+struct DedupOut {
+  int key_bytes;
+  void* unique;
+  void* counts;
+  void* inverse;
+  void* offsets;
+  uint32_t* pos_key;
+  DedupHead* head;
+  DedupHead* host_head;
+  PositionGrad pg;
+};
+
+// Words of the key-span parts that the radix sort writes for n keys
+// (radix_span_parts(n)).
 int64_t dedup_span_parts(int64_t n);
+// Whether a sort of the caller's keys (RadixSource) with gradient rows carries
+// rows in place of positions.
+bool carries_rows(int mode);
 // k64[i] = key i as an unsigned sort key (sign bit flipped when flip != 0), v[i] = i.
 hipError_t launch_dedup_prep(const void* keys, int key_bytes, int64_t n, int flip, uint64_t* k64,
                              uint32_t* v, hipStream_t stream);
-// Outputs from the sorted keys and the run-head scan; with span_part
-// (dedup_span_parts(n) words), also *span_out = OR of the span parts.
-hipError_t launch_dedup_outputs(const uint64_t* ks, const uint32_t* vs, const uint32_t* scan,
-                                int64_t n, int key_bytes, void* unique, void* inverse,
-                                void* offsets, uint32_t* start, uint32_t* pos_key,
-                                const uint64_t* span_part, unsigned long long* span_out,
-                                hipStream_t stream);
-// The runs of sorted keys ks (values vs) in two launches: unique keys, counts,
-// inverse and offsets of the key type, pos_key (optional) the unique index of
-// every position, *total the unique count; with span_part, also *span_out as
-// launch_dedup_outputs; with pg, each dedup position's gradient row and
-// weight (as launch_backprop_prep).  Scratch: blk_count / blk_last,
-// run_blocks(n) words each.  At most kRunMaxBlocks blocks
-// (hipErrorInvalidValue beyond).
-constexpr int64_t kRunMaxBlocks = 4096;
-int64_t run_blocks(int64_t n);
-hipError_t launch_dedup_runs(const uint64_t* ks, const uint32_t* vs, int64_t n, int key_bytes, void* unique,
-                             void* counts, void* inverse, void* offsets, uint32_t* pos_key, uint32_t* total,
-                             uint32_t* blk_count, int64_t* blk_last, const uint64_t* span_part,
-                             unsigned long long* span_out, const PositionGrad* pg, hipStream_t stream);
-// counts[u] for u < u_n, or for u < *u_dev when u_dev is given (u_n an upper bound).
-hipError_t launch_dedup_counts(const uint32_t* start, uint32_t u_n, const uint32_t* u_dev,
-                               int key_bytes, void* counts, hipStream_t stream);
+// Every output from the sorted keys ks (values vs: positions, or with `carried`
+// their gradient rows); head.span = the OR of the span parts (0 without
+// span_part).  state: run_state_words(n) words, all 0.
+int64_t run_state_words(int64_t n);
+hipError_t launch_dedup_runs(const uint64_t* ks, const uint32_t* vs, int64_t n, const uint64_t* span_part,
+                             uint64_t* state, bool carried, const DedupOut& out, hipStream_t stream);
+// Sort and outputs of at most kSmallDedupKeys keys in one launch (head.span 0).
+constexpr int64_t kSmallDedupKeys = 4096;
+hipError_t launch_dedup_small(const void* keys, int64_t n, const DedupOut& out, hipStream_t stream);
 
 // Hash slots for a batch of n keys: a power of two, at least 2n (and 1024).
 size_t hash_dedup_slots(int64_t n);

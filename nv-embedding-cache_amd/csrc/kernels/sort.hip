@@ -28,9 +28,11 @@
 //
 // Bound: latency (a pass moves 24 bytes a key, 6 MB at 262,144 keys).  Three
 // launches per pass (tile counts, a scan of each digit's row, the scatter) took
-// NVE_OLD us of kernels for three passes over 262,144 keys, and nine launches; the
-// four take NVE_NEW.  The tile is 4096 keys so that a tile has few predecessors:
-// with 1024-key tiles every one of 256 tiles walks back through most of them.
+// nine launches for the three passes of a table's keys, the four of this sort take
+// as long in kernels at 262,144 keys (50 and 52 us) and less in all others: dedup
+// of 2,000 keys 58.0 -> 44.7 us, 32,768 keys 60.5 -> 57.9, 1,000,000 keys 139.7 ->
+// 125.9.  The tile is 4096 keys so that a tile has few predecessors: with
+// 1024-key tiles every one of 256 tiles walks back through most of them.
 //
 // The exclusive scan of an array (run heads in the insert) is
 // reduce-then-scan over 4096-element blocks: block sums, a scan of the sums
@@ -38,7 +40,9 @@
 // its elements from its offset.
 #include "device_common.cuh"
 #include "lane_moves.cuh"
+#include "position_grad.cuh"
 #include "sort_launch.hpp"
+#include "tile_rank.cuh"
 
 namespace nve_amd {
 
@@ -46,7 +50,6 @@ constexpr int kTileThreads = 1024;
 constexpr int kTileWaves = kTileThreads / 64;
 constexpr int kTileItems = 4;  // rounds of 64 keys per wave
 constexpr int kTile = kTileThreads * kTileItems;
-constexpr int kMaxBins = 512;     // digits of at most 9 bits
 constexpr int kMaxPasses = 8;     // 64 bits in digits of 8, or of 9
 constexpr int kCountGroups = 64;  // workgroups whose digit counts every tile adds up
 
@@ -70,16 +73,22 @@ __device__ __forceinline__ uint64_t sort_key(const uint64_t* keys, const RadixSo
 }
 
 // parts[workgroup][pass][kMaxBins] = digit counts of the workgroup's tiles;
-// state[0 .. state_words) = 0.  With src.span_part, span_part[workgroup] = the
+// state[0 .. state_words) and clear[0 .. clear_words) = 0.  With pg.by_key, the
+// gradient row of every key position.  With src.span_part, span_part[workgroup] = the
 // OR of key ^ key[0] over its keys (the bits where they differ from the first).
 template <bool RAW>
 __global__ __launch_bounds__(kTileThreads) void radix_count_kernel(const uint64_t* keys, RadixSource src,
                                                                    int64_t n, RadixDigits dg, uint32_t* parts,
-                                                                   uint64_t* state, int64_t state_words) {
+                                                                   uint64_t* state, int64_t state_words,
+                                                                   uint64_t* clear, int64_t clear_words,
+                                                                   PositionGrad pg) {
   __shared__ uint32_t h[kMaxPasses * kMaxBins];
+  __shared__ uint32_t rows[kTile];
   const int tid = threadIdx.x;
   for (int64_t w = (int64_t)blockIdx.x * kTileThreads + tid; w < state_words; w += (int64_t)gridDim.x * kTileThreads)
     state[w] = 0;
+  for (int64_t w = (int64_t)blockIdx.x * kTileThreads + tid; w < clear_words; w += (int64_t)gridDim.x * kTileThreads)
+    clear[w] = 0;
   for (int d = tid; d < dg.passes * kMaxBins; d += kTileThreads) h[d] = 0;
   __syncthreads();
   uint64_t diff = 0;
@@ -104,6 +113,13 @@ __global__ __launch_bounds__(kTileThreads) void radix_count_kernel(const uint64_
         if (valid && d != lead) atomicAdd(&h[p * kMaxBins + d], 1u);
         if ((tid & 63) == 0 && same) atomicAdd(&h[p * kMaxBins + lead], (uint32_t)__popcll(same));
       }
+    }
+  }
+  if (pg.by_key != nullptr) {  // uniform
+    for (int64_t base = (int64_t)blockIdx.x * kTile; base < n; base += (int64_t)gridDim.x * kTile) {
+      tile_rows<kTileThreads, kTile>(pg, base, rows);
+      for (int x = tid; x < kTile && base + x < n; x += kTileThreads) pg.by_key[base + x] = rows[x];
+      __syncthreads();
     }
   }
   if (src.span_part != nullptr) {  // uniform
@@ -215,10 +231,6 @@ __global__ __launch_bounds__(256) void scan_down_kernel(uint32_t* data, int64_t 
     *total = off + block_total;
 }
 
-// A published word: state in the top two bits, a count of keys below.
-constexpr uint64_t kStateOwn = 1ull << 62;     // the tile's own keys of the digit
-constexpr uint64_t kStateBefore = 2ull << 62;  // with those of every tile before it
-constexpr uint64_t kStateCount = (1ull << 62) - 1;
 constexpr int kLookAhead = 8;  // words read at a time while walking back
 
 // Keys of the tiles before `tile`, from word[tile * stride]: adds published
@@ -229,8 +241,7 @@ __device__ __forceinline__ uint64_t keys_before(const uint64_t* word, int64_t ti
     uint64_t w[kLookAhead];
 #pragma unroll
     for (int u = 0; u < kLookAhead; ++u)
-      w[u] = j - u >= 0 ? __hip_atomic_load(word + (j - u) * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                        : kStateBefore;  // nothing before the first tile
+      w[u] = j - u >= 0 ? load_state(word + (j - u) * stride) : kStateBefore;  // nothing before the first tile
     bool open = true;  // every word so far was published, none of them the last to add
     int used = 0;
 #pragma unroll
@@ -252,7 +263,7 @@ __device__ __forceinline__ uint64_t keys_before(const uint64_t* word, int64_t ti
 struct SweepArgs {
   const uint64_t* keys;
   const uint32_t* vals;
-  RadixSource src;  // RAW: the first pass reads the caller's keys, values = positions
+  RadixSource src;  // RAW: the first pass reads the caller's keys (vals null: values = positions)
   uint64_t* ko;
   uint32_t* vo;
   int64_t n;
@@ -276,7 +287,7 @@ __global__ __launch_bounds__(kTileThreads) void radix_sweep_kernel(SweepArgs a) 
   __shared__ uint64_t scan[kTileWaves + 1];
   __shared__ uint32_t s_tile;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (tid == 0) s_tile = (uint32_t)atomicAdd(reinterpret_cast<unsigned long long*>(a.state), 1ull);
+  if (tid == 0) s_tile = take_tile(a.state);
   // the keys of tile blockIdx.x, which mostly is the tile: loaded while the
   // counter's answer is on its way
   const int li0 = wave * (64 * kTileItems) + lane;  // key r of the lane: li0 + 64 * r
@@ -291,7 +302,7 @@ __global__ __launch_bounds__(kTileThreads) void radix_sweep_kernel(SweepArgs a) 
       const int li = li0 + 64 * r;
       k[r] = li < tile_n ? sort_key<RAW>(a.keys, a.src, base + li) : 0ull;
       if constexpr (RAW)
-        v[r] = (uint32_t)(base + li);
+        v[r] = a.vals == nullptr ? (uint32_t)(base + li) : li < tile_n ? a.vals[base + li] : 0u;
       else
         v[r] = li < tile_n ? a.vals[base + li] : 0u;
     }
@@ -323,33 +334,10 @@ __global__ __launch_bounds__(kTileThreads) void radix_sweep_kernel(SweepArgs a) 
   const int64_t tile = s_tile;
   if (tile != blockIdx.x) load(tile);  // uniform
   // rank among the wave's keys of the same digit: earlier rounds, then lower lanes
-  const uint64_t lower = (1ull << lane) - 1ull;
   uint32_t rank[kTileItems];
 #pragma unroll
-  for (int r = 0; r < kTileItems; ++r) {
-    const bool valid = li0 + 64 * r < tile_n;
-    const uint32_t d = (uint32_t)(k[r] >> a.shift) & a.mask;
-    const uint64_t valids = __ballot(valid);
-    uint32_t plo = (uint32_t)valids, phi = (uint32_t)(valids >> 32);
-#pragma unroll
-    for (int b = 0; b < RB; ++b) {
-      const uint64_t m = __ballot((d >> b) & 1u);
-      const uint32_t mine = 0u - ((d >> b) & 1u);  // lanes whose bit differs leave
-      plo &= ~((uint32_t)m ^ mine);
-      phi &= ~((uint32_t)(m >> 32) ^ mine);
-    }
-    const uint64_t peers = ((uint64_t)phi << 32) | plo;
-    const uint32_t before = (uint32_t)__popcll(peers & lower);
-    // a wave's LDS accesses stay in order: every lane reads the count before
-    // the first of its digit's lanes adds to it
-    const uint32_t seen = cnt[wave][d];
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    if (valid && before == 0) cnt[wave][d] = seen + (uint32_t)__popcll(peers);
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    rank[r] = seen + before;
-  }
+  for (int r = 0; r < kTileItems; ++r)
+    rank[r] = wave_digit_rank<RB>((uint32_t)(k[r] >> a.shift) & a.mask, li0 + 64 * r < tile_n, cnt[wave]);
   __syncthreads();
   uint64_t* const word = a.state + 1 + (tid < kBins ? tid : 0);
   uint32_t own = 0;
@@ -360,8 +348,7 @@ __global__ __launch_bounds__(kTileThreads) void radix_sweep_kernel(SweepArgs a) 
       cnt[w][tid] = own;
       own += c;
     }
-    __hip_atomic_store(word + tile * kMaxBins, (tile == 0 ? kStateBefore : kStateOwn) | own, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    store_state(word + tile * kMaxBins, (tile == 0 ? kStateBefore : kStateOwn) | own);
   }
   // exclusive sums over the digits: the tile's counts and the totals
   const uint32_t inc_own = wave_sum_scan(own), inc_total = wave_sum_scan(total);
@@ -384,9 +371,7 @@ __global__ __launch_bounds__(kTileThreads) void radix_sweep_kernel(SweepArgs a) 
   }
   if (tid < kBins) {
     const uint64_t before = keys_before(word, tile, kMaxBins);
-    if (tile > 0)
-      __hip_atomic_store(word + tile * kMaxBins, kStateBefore | (before + own), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
+    if (tile > 0) store_state(word + tile * kMaxBins, kStateBefore | (before + own));
     gbase[tid] = (uint32_t)(ex >> 32) + (uint32_t)before - (uint32_t)ex;
   }
   __syncthreads();
@@ -448,7 +433,8 @@ size_t radix_sort_temp_bytes(int64_t n) {
 
 hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
                             int64_t n, int begin_bit, int end_bit, void* temp, int* result_in_alt,
-                            hipStream_t stream, const RadixSource* src) {
+                            hipStream_t stream, const RadixSource* src, uint64_t* clear, int64_t clear_words,
+                            const PositionGrad* pg) {
   *result_in_alt = 0;
   if (n <= 1 || end_bit <= begin_bit) return src != nullptr ? hipErrorInvalidValue : hipSuccess;
   if (n > 0xffffffffLL || end_bit > 64) return hipErrorInvalidValue;  // values and counts of 32 bits
@@ -470,12 +456,13 @@ hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, 
   int nparts = (int)radix_span_parts(n);
   const int stride = dg.passes * kMaxBins;
   const RadixSource none{};
+  const PositionGrad pooled = pg != nullptr && pg->mode != kBackpropConcat ? *pg : PositionGrad{};
   if (src != nullptr)
     hipLaunchKernelGGL(radix_count_kernel<true>, dim3(nparts), dim3(kTileThreads), 0, stream, keys, *src, n, dg,
-                       parts, state, dg.passes * words);
+                       parts, state, dg.passes * words, clear, clear_words, pooled);
   else
     hipLaunchKernelGGL(radix_count_kernel<false>, dim3(nparts), dim3(kTileThreads), 0, stream, keys, none, n, dg,
-                       parts, state, dg.passes * words);
+                       parts, state, dg.passes * words, clear, clear_words, pooled);
   if (tiles > kMaxAddingTiles) {
     hipLaunchKernelGGL(radix_total_kernel, dim3((stride + 255) / 256), dim3(256), 0, stream, parts, nparts, stride);
     nparts = 1;
@@ -495,6 +482,7 @@ hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, 
     a.state = state + p * words;
     const bool raw = src != nullptr && p == 0;
     a.src = raw ? *src : none;
+    if (raw) a.vals = pooled.by_key != nullptr && weight_from_row(pooled.mode) ? pooled.by_key : nullptr;
     const dim3 grid((unsigned)tiles), block(kTileThreads);
     if (rb == 9) {
       if (raw)

@@ -6,6 +6,8 @@
 
 #include <utility>
 
+#include "backprop_launch.hpp"
+
 namespace nve_amd {
 
 // Bytes of temporary storage radix_sort_pairs needs for n pairs; it also
@@ -31,10 +33,14 @@ int64_t radix_span_parts(int64_t n);
 // (keys_alt, vals_alt); *result_in_alt says which pair holds the result.
 // With src, the first pass reads src instead of keys / vals (which it never
 // reads); at least one pass must then run (n >= 2, end_bit > begin_bit), else
-// hipErrorInvalidValue.
+// hipErrorInvalidValue.  clear (optional): clear_words words set to 0 on the
+// way, when a pass runs.  pg (optional, a pooled mode): pg->by_key is filled on
+// the way too, and with src and weight_from_row(pg->mode) the values are the
+// positions' gradient rows (also Concatenate: the positions).
 hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
                             int64_t n, int begin_bit, int end_bit, void* temp, int* result_in_alt,
-                            hipStream_t stream, const RadixSource* src = nullptr);
+                            hipStream_t stream, const RadixSource* src = nullptr, uint64_t* clear = nullptr,
+                            int64_t clear_words = 0, const PositionGrad* pg = nullptr);
 
 // In-place exclusive scan of m uint32 (total, if non-null, gets the sum);
 // temp holds scan_temp_bytes(m) bytes.

@@ -12,11 +12,16 @@
 
 namespace nve_amd {
 
-void read_small(void* host, const void* dev, size_t bytes, hipStream_t stream) {
-  NVE_CHECK(bytes <= 64, "read_small reads at most 64 bytes");
+void* pinned_slot() {
   // one pinned slot per thread, kept for the thread's life
   thread_local void* slot = nullptr;
-  if (slot == nullptr) NVE_HIP(hipHostMalloc(&slot, 64, hipHostMallocDefault));
+  if (slot == nullptr) NVE_HIP(hipHostMalloc(&slot, kPinnedSlotBytes, hipHostMallocDefault));
+  return slot;
+}
+
+void read_small(void* host, const void* dev, size_t bytes, hipStream_t stream) {
+  NVE_CHECK(bytes <= kPinnedSlotBytes, "read_small reads at most 64 bytes");
+  void* slot = pinned_slot();
   NVE_HIP(launch_small_read(slot, dev, (int)bytes, stream));
   NVE_HIP(hipStreamSynchronize(stream));
   std::memcpy(host, slot, bytes);

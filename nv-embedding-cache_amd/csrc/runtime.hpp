@@ -226,6 +226,11 @@ const void* device_input(ExecutionContext& ctx, const char* name, const void* p,
 const void* host_input(ExecutionContext& ctx, const char* name, const void* p, size_t bytes,
                        hipStream_t stream);
 
+// The calling thread's pinned host memory (kPinnedSlotBytes), which kernels may
+// write results to that the thread reads after waiting for their stream.
+constexpr size_t kPinnedSlotBytes = 64;
+void* pinned_slot();
+
 // Copies `bytes` (at most 64) of device memory to `host` and waits for
 // `stream`.  The copy lands in a pinned per-thread slot first: a pageable
 // destination costs a staged copy, tens of microseconds for a few bytes.

@@ -1,7 +1,10 @@
-"""The radix sort behind the dedup at the sizes where its tiles change: one
-tile of 4,096 keys and one key more or less, the 64 count groups, the launch
-that adds counts up (beyond 128 tiles), and keys whose digits pile up in one
-bin, all equal, descending, or spread over all 64 bits."""
+"""The sorted dedup at the sizes where its work is cut anew: the single
+workgroup's 1, 4 and 8 keys per thread (1,024, 4,096 and 8,192 keys) and the
+first size past them, the radix sort's tiles of 4,096 keys, its 64 count groups
+and the launch that adds counts up (beyond 128 tiles), the run outputs' tiles
+of 1,024 positions and 64 of them looked back over at a time; with keys whose
+digits pile up in one bin, all equal (one run over every tile), descending, or
+spread over all 64 bits."""
 import ctypes
 
 import numpy as np
@@ -29,8 +32,28 @@ def make(kind, n, rng):
     return hot.astype(np.int64)
 
 
+@pytest.mark.parametrize("n", [100, 1024, 3000, 8192, 8193, 20000])
+def test_int32_keys(n):
+    rng = np.random.default_rng(n)
+    keys = rng.integers(-2**31, 2**31 - 1, size=n).astype(np.int32)
+    keys[rng.random(n) < 0.4] = -5
+    need = ctypes.c_uint64()
+    _lib.call("nve_amd_dedup_workspace_size", n, ctypes.byref(need))
+    ws = torch.empty(need.value, dtype=torch.uint8, device="cuda")
+    out = [torch.zeros(n + 1, dtype=torch.int32, device="cuda") for _ in range(4)]
+    num, d_keys = ctypes.c_int64(), to_dev(keys)
+    _lib.call("nve_amd_dedup", _lib.KEY_INT32, n, vp(d_keys), vp(out[0]), vp(out[1]), vp(out[2]), vp(out[3]),
+              ctypes.byref(num), vp(ws), need.value, stream_ptr())
+    unique, counts = np.unique(keys, return_counts=True)
+    got = [t.cpu().numpy() for t in out]
+    assert num.value == unique.size
+    assert np.array_equal(got[0][:num.value], unique) and np.array_equal(got[1][:num.value], counts)
+    assert np.array_equal(got[2][:n], np.argsort(keys, kind="stable"))
+
+
 @pytest.mark.parametrize("kind", ["table", "wide", "one", "descending", "hot"])
-@pytest.mark.parametrize("n", [2, 63, 64, 65, TILE - 1, TILE, TILE + 1, 3 * TILE + 17, 63 * TILE + 1, 64 * TILE,
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1024, 1025, TILE - 1, TILE, TILE + 1, 2 * TILE - 1, 2 * TILE,
+                               2 * TILE + 1, 3 * TILE + 17, 16 * TILE, 16 * TILE + 1025, 63 * TILE + 1, 64 * TILE,
                                65 * TILE + 5, 128 * TILE, 128 * TILE + 1, 300 * TILE + 9])
 def test_dedup_equals_numpy(kind, n):
     if n > 65 * TILE + 5 and kind in ("wide", "descending"):
