@@ -13,9 +13,9 @@
 // keys.  Digits have 8 bits, or 9 when that takes fewer passes (the last digit
 // keeps only the bits below end_bit).
 //   count    at most kCountGroups workgroups, each the digit counts of its
-//            4096-key tiles for every pass; it also clears the passes' state;
-//   sweep    a 1024-thread workgroup per 4096-key tile.  A wave ranks its 256
-//            keys with one ballot per digit bit and a running count per digit
+//            tiles for every pass; it also clears the passes' state;
+//   sweep    a 1024-thread workgroup per tile of 2,048 or 4,096 keys.  A wave ranks
+//            its keys with one ballot per digit bit and a running count per digit
 //            in LDS; the tile's counts are published, the tile is staged in LDS
 //            in digit order, and each digit's place is found from the tiles
 //            before: their published counts are added, walking back until one
@@ -28,16 +28,21 @@
 //
 // Bound: latency (a pass moves 24 bytes a key, 6 MB at 262,144 keys).  Three
 // launches per pass (tile counts, a scan of each digit's row, the scatter) took
-// nine launches for the three passes of a table's keys, the four of this sort take
-// as long in kernels at 262,144 keys (50 and 52 us) and less in all others: dedup
-// of 2,000 keys 58.0 -> 44.7 us, 32,768 keys 60.5 -> 57.9, 1,000,000 keys 139.7 ->
-// 125.9.  The tile is 4096 keys so that a tile has few predecessors: with
-// 1024-key tiles every one of 256 tiles walks back through most of them.
+// nine launches for the three passes of a table's keys; the four of this sort and
+// the one launch of the dedup's runs take the dedup of 8,192 keys from 67 to 44 us,
+// of 32,768 keys from 66 to 51, of 131,072 keys from 67 to 61.5, of 262,144 keys from 73 to 73
+// and of 1,000,000 keys from 122 to 109.  Tiles are large so that each has few
+// predecessors: with 1024-key tiles every one of 256 tiles walks back through most
+// of them.  Nor do more words per step of the walk help (kLookAhead 8, 16 and 32:
+// 262,144 keys 73.5, 75.0 and 77.4 us): the walk is bound by the words it reads.
 //
 // The exclusive scan of an array (run heads in the insert) is
 // reduce-then-scan over 4096-element blocks: block sums, a scan of the sums
 // (recursively, in the caller's temporary storage), then each block rescans
 // its elements from its offset.
+#include <algorithm>
+#include <type_traits>
+
 #include "device_common.cuh"
 #include "lane_moves.cuh"
 #include "position_grad.cuh"
@@ -48,8 +53,7 @@ namespace nve_amd {
 
 constexpr int kTileThreads = 1024;
 constexpr int kTileWaves = kTileThreads / 64;
-constexpr int kTileItems = 4;  // rounds of 64 keys per wave
-constexpr int kTile = kTileThreads * kTileItems;
+constexpr int kCountTile = 2 * kTileThreads;  // keys a counting workgroup has at least
 constexpr int kMaxPasses = 8;     // 64 bits in digits of 8, or of 9
 constexpr int kCountGroups = 64;  // workgroups whose digit counts every tile adds up
 
@@ -76,12 +80,13 @@ __device__ __forceinline__ uint64_t sort_key(const uint64_t* keys, const RadixSo
 // state[0 .. state_words) and clear[0 .. clear_words) = 0.  With pg.by_key, the
 // gradient row of every key position.  With src.span_part, span_part[workgroup] = the
 // OR of key ^ key[0] over its keys (the bits where they differ from the first).
-template <bool RAW>
+template <bool RAW, int ITEMS>
 __global__ __launch_bounds__(kTileThreads) void radix_count_kernel(const uint64_t* keys, RadixSource src,
                                                                    int64_t n, RadixDigits dg, uint32_t* parts,
                                                                    uint64_t* state, int64_t state_words,
                                                                    uint64_t* clear, int64_t clear_words,
                                                                    PositionGrad pg) {
+  constexpr int kTile = kTileThreads * ITEMS;
   __shared__ uint32_t h[kMaxPasses * kMaxBins];
   __shared__ uint32_t rows[kTile];
   const int tid = threadIdx.x;
@@ -94,14 +99,14 @@ __global__ __launch_bounds__(kTileThreads) void radix_count_kernel(const uint64_
   uint64_t diff = 0;
   const uint64_t k0 = sort_key<RAW>(keys, src, 0);
   for (int64_t base = (int64_t)blockIdx.x * kTile; base < n; base += (int64_t)gridDim.x * kTile) {
-    uint64_t k[kTileItems];
+    uint64_t k[ITEMS];
 #pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
       const int64_t i = base + r * kTileThreads + tid;
       k[r] = sort_key<RAW>(keys, src, i < n ? i : 0);
     }
 #pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
       const bool valid = base + r * kTileThreads + tid < n;
       diff |= k[r] ^ k0;  // a lane past the end holds key 0
       for (int p = 0; p < dg.passes; ++p) {
@@ -275,9 +280,10 @@ struct SweepArgs {
   uint64_t* state;  // the pass's words: tile counter, then kMaxBins per tile
 };
 
-template <int RB, bool RAW>
+template <int RB, bool RAW, int ITEMS>
 __global__ __launch_bounds__(kTileThreads) void radix_sweep_kernel(SweepArgs a) {
   constexpr int kBins = 1 << RB;
+  constexpr int kTile = kTileThreads * ITEMS;
   static_assert(kBins <= kTileThreads && kBins <= kMaxBins, "one thread per digit");
   __shared__ uint64_t sk[kTile];
   __shared__ uint32_t sv[kTile];
@@ -290,15 +296,15 @@ __global__ __launch_bounds__(kTileThreads) void radix_sweep_kernel(SweepArgs a) 
   if (tid == 0) s_tile = take_tile(a.state);
   // the keys of tile blockIdx.x, which mostly is the tile: loaded while the
   // counter's answer is on its way
-  const int li0 = wave * (64 * kTileItems) + lane;  // key r of the lane: li0 + 64 * r
-  uint64_t k[kTileItems];
-  uint32_t v[kTileItems];
+  const int li0 = wave * (64 * ITEMS) + lane;  // key r of the lane: li0 + 64 * r
+  uint64_t k[ITEMS];
+  uint32_t v[ITEMS];
   int tile_n;
   const auto load = [&](int64_t t) {
     const int64_t base = t * kTile;
     tile_n = (int)(a.n - base < kTile ? a.n - base : kTile);
 #pragma unroll
-    for (int r = 0; r < kTileItems; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
       const int li = li0 + 64 * r;
       k[r] = li < tile_n ? sort_key<RAW>(a.keys, a.src, base + li) : 0ull;
       if constexpr (RAW)
@@ -334,9 +340,9 @@ __global__ __launch_bounds__(kTileThreads) void radix_sweep_kernel(SweepArgs a) 
   const int64_t tile = s_tile;
   if (tile != blockIdx.x) load(tile);  // uniform
   // rank among the wave's keys of the same digit: earlier rounds, then lower lanes
-  uint32_t rank[kTileItems];
+  uint32_t rank[ITEMS];
 #pragma unroll
-  for (int r = 0; r < kTileItems; ++r)
+  for (int r = 0; r < ITEMS; ++r)
     rank[r] = wave_digit_rank<RB>((uint32_t)(k[r] >> a.shift) & a.mask, li0 + 64 * r < tile_n, cnt[wave]);
   __syncthreads();
   uint64_t* const word = a.state + 1 + (tid < kBins ? tid : 0);
@@ -361,7 +367,7 @@ __global__ __launch_bounds__(kTileThreads) void radix_sweep_kernel(SweepArgs a) 
   if (tid < kBins) lstart[tid] = (uint32_t)ex;
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kTileItems; ++r) {
+  for (int r = 0; r < ITEMS; ++r) {
     if (li0 + 64 * r < tile_n) {
       const uint32_t d = (uint32_t)(k[r] >> a.shift) & a.mask;
       const uint32_t pos = lstart[d] + cnt[wave][d] + rank[r];
@@ -416,16 +422,32 @@ size_t scan_temp_bytes(int64_t m) {
 }
 
 namespace {
-int64_t tiles_of(int64_t n) { return n > 0 ? (n + kTile - 1) / kTile : 1; }
-int64_t pass_words(int64_t n) { return 1 + tiles_of(n) * kMaxBins; }
+// Rounds of 64 keys per wave, and so the tile of a sweep (1,024 keys per round).
+// Two rounds halve a tile's chain of ranking rounds and double the workgroups
+// where 4,096-key tiles leave most CUs idle, but past 64 tiles a tile walks back
+// over too many others.  Dedup with two and with four rounds: 8,192 keys 44.0 and 51.0 us,
+// 32,768 keys 50.8 and 56.5, 131,072 keys 61.5 and 64.4, 262,144 keys 79.0 and
+// 73.5, 1,000,000 keys 151 and 110.  (One round up to 16,384 keys: within 0.3 us of two.)
+constexpr int64_t kTwoRoundKeys = 131072;
+int tile_items(int64_t n) { return n <= kTwoRoundKeys ? 2 : 4; }
+int64_t tiles_of(int64_t n) {
+  const int64_t tile = kTileThreads * tile_items(n);
+  return n > 0 ? (n + tile - 1) / tile : 1;
+}
+// The most tiles of any batch of at most n keys: storage sized for n serves them all.
+int64_t most_tiles(int64_t n) { return std::max(tiles_of(n), tiles_of(std::min(n, kTwoRoundKeys))); }
+int64_t pass_words(int64_t tiles) { return 1 + tiles * kMaxBins; }
 // past this many tiles one launch adds the counts up
 constexpr int64_t kMaxAddingTiles = 128;
 }  // namespace
 
-int64_t radix_span_parts(int64_t n) { return tiles_of(n) < kCountGroups ? tiles_of(n) : kCountGroups; }
+int64_t radix_span_parts(int64_t n) {
+  const int64_t groups = n > 0 ? (n + kCountTile - 1) / kCountTile : 1;
+  return groups < kCountGroups ? groups : kCountGroups;
+}
 
 size_t radix_sort_temp_bytes(int64_t n) {
-  const size_t sort = (size_t)kMaxPasses * (size_t)pass_words(n) * 8 +
+  const size_t sort = (size_t)kMaxPasses * (size_t)pass_words(most_tiles(n)) * 8 +
                       (size_t)radix_span_parts(n) * kMaxPasses * kMaxBins * 4;
   const size_t scan = scan_temp_bytes(n);
   return sort > scan ? sort : scan;
@@ -451,18 +473,22 @@ hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, 
     ++dg.passes;
   }
   uint64_t* state = static_cast<uint64_t*>(temp);
-  const int64_t words = pass_words(n);
+  const int64_t words = pass_words(tiles);
   uint32_t* parts = reinterpret_cast<uint32_t*>(state + (int64_t)dg.passes * words);
   int nparts = (int)radix_span_parts(n);
   const int stride = dg.passes * kMaxBins;
   const RadixSource none{};
   const PositionGrad pooled = pg != nullptr && pg->mode != kBackpropConcat ? *pg : PositionGrad{};
-  if (src != nullptr)
-    hipLaunchKernelGGL(radix_count_kernel<true>, dim3(nparts), dim3(kTileThreads), 0, stream, keys, *src, n, dg,
-                       parts, state, dg.passes * words, clear, clear_words, pooled);
-  else
-    hipLaunchKernelGGL(radix_count_kernel<false>, dim3(nparts), dim3(kTileThreads), 0, stream, keys, none, n, dg,
-                       parts, state, dg.passes * words, clear, clear_words, pooled);
+  const int items = tile_items(n);
+#define NVE_LAUNCH_COUNT(RAW, ITEMS, SRC)                                                                         \
+  hipLaunchKernelGGL((radix_count_kernel<RAW, ITEMS>), dim3(nparts), dim3(kTileThreads), 0, stream, keys, SRC, n, \
+                     dg, parts, state, dg.passes * words, clear, clear_words, pooled)
+  if (src != nullptr) {
+    if (items == 2) NVE_LAUNCH_COUNT(true, 2, *src); else NVE_LAUNCH_COUNT(true, 4, *src);
+  } else {
+    if (items == 2) NVE_LAUNCH_COUNT(false, 2, none); else NVE_LAUNCH_COUNT(false, 4, none);
+  }
+#undef NVE_LAUNCH_COUNT
   if (tiles > kMaxAddingTiles) {
     hipLaunchKernelGGL(radix_total_kernel, dim3((stride + 255) / 256), dim3(256), 0, stream, parts, nparts, stride);
     nparts = 1;
@@ -484,17 +510,19 @@ hipError_t radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, 
     a.src = raw ? *src : none;
     if (raw) a.vals = pooled.by_key != nullptr && weight_from_row(pooled.mode) ? pooled.by_key : nullptr;
     const dim3 grid((unsigned)tiles), block(kTileThreads);
-    if (rb == 9) {
-      if (raw)
-        hipLaunchKernelGGL((radix_sweep_kernel<9, true>), grid, block, 0, stream, a);
+    const auto sweep = [&](auto IT) {
+      constexpr int kItems = decltype(IT)::value;
+      if (rb == 9 && raw)
+        hipLaunchKernelGGL((radix_sweep_kernel<9, true, kItems>), grid, block, 0, stream, a);
+      else if (rb == 9)
+        hipLaunchKernelGGL((radix_sweep_kernel<9, false, kItems>), grid, block, 0, stream, a);
+      else if (raw)
+        hipLaunchKernelGGL((radix_sweep_kernel<8, true, kItems>), grid, block, 0, stream, a);
       else
-        hipLaunchKernelGGL((radix_sweep_kernel<9, false>), grid, block, 0, stream, a);
-    } else {
-      if (raw)
-        hipLaunchKernelGGL((radix_sweep_kernel<8, true>), grid, block, 0, stream, a);
-      else
-        hipLaunchKernelGGL((radix_sweep_kernel<8, false>), grid, block, 0, stream, a);
-    }
+        hipLaunchKernelGGL((radix_sweep_kernel<8, false, kItems>), grid, block, 0, stream, a);
+    };
+    if (items == 2) sweep(std::integral_constant<int, 2>{});
+    else sweep(std::integral_constant<int, 4>{});
     a.keys = p & 1 ? keys : keys_alt;
     a.vals = p & 1 ? vals : vals_alt;
     a.ko = p & 1 ? keys_alt : keys;
