@@ -30,11 +30,12 @@
 // launches per pass (tile counts, a scan of each digit's row, the scatter) took
 // nine launches for the three passes of a table's keys; the four of this sort and
 // the one launch of the dedup's runs take the dedup of 8,192 keys from 67 to 44 us,
-// of 32,768 keys from 66 to 51, of 131,072 keys from 67 to 61.5, of 262,144 keys from 73 to 73
-// and of 1,000,000 keys from 122 to 109.  Tiles are large so that each has few
+// of 32,768 keys from 66 to 51, of 131,072 keys from 67 to 61, of 262,144 keys from 73 to 71
+// and of 1,000,000 keys from 122 to 108.  Tiles are large so that each has few
 // predecessors: with 1024-key tiles every one of 256 tiles walks back through most
-// of them.  Nor do more words per step of the walk help (kLookAhead 8, 16 and 32:
-// 262,144 keys 73.5, 75.0 and 77.4 us): the walk is bound by the words it reads.
+// of them.  Nor do more words per step of the walk help (4,096-key tiles, 1,000,000 keys:
+// kLookAhead 4, 8, 16 and 32 take 107.6, 109.5, 112 and 118 us): the walk is bound
+// by the words it reads.
 //
 // The exclusive scan of an array (run heads in the insert) is
 // reduce-then-scan over 4096-element blocks: block sums, a scan of the sums
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(256) void scan_down_kernel(uint32_t* data, int64_t 
     *total = off + block_total;
 }
 
-constexpr int kLookAhead = 8;  // words read at a time while walking back
+constexpr int kLookAhead = 4;  // words read at a time while walking back
 
 // Keys of the tiles before `tile`, from word[tile * stride]: adds published
 // counts from tile - 1 down until one that includes all before it.
@@ -424,11 +425,12 @@ size_t scan_temp_bytes(int64_t m) {
 namespace {
 // Rounds of 64 keys per wave, and so the tile of a sweep (1,024 keys per round).
 // Two rounds halve a tile's chain of ranking rounds and double the workgroups
-// where 4,096-key tiles leave most CUs idle, but past 64 tiles a tile walks back
-// over too many others.  Dedup with two and with four rounds: 8,192 keys 44.0 and 51.0 us,
-// 32,768 keys 50.8 and 56.5, 131,072 keys 61.5 and 64.4, 262,144 keys 79.0 and
-// 73.5, 1,000,000 keys 151 and 110.  (One round up to 16,384 keys: within 0.3 us of two.)
-constexpr int64_t kTwoRoundKeys = 131072;
+// where 4,096-key tiles leave most CUs idle, but past 128 tiles a tile walks back
+// over too many others.  Dedup with two and with four rounds (8 words per step of the
+// walk): 8,192 keys 44.4 and 51.0 us, 32,768 keys 50.8 and 56.5, 131,072 keys 61.6
+// and 64.4, 262,144 keys 72.2 and 73.2, 1,000,000 keys 127 and 109.  (One round up to
+// 16,384 keys: within 0.3 us of two at 8,192 and 16,384 keys, 1.4 us less at 5,000.)
+constexpr int64_t kTwoRoundKeys = 262144;
 int tile_items(int64_t n) { return n <= kTwoRoundKeys ? 2 : 4; }
 int64_t tiles_of(int64_t n) {
   const int64_t tile = kTileThreads * tile_items(n);

@@ -1,6 +1,6 @@
 """The sorted dedup at the sizes where its work is cut anew: the single
 workgroup's 1 and 4 keys per thread (1,024 and 4,096 keys) and the
-first size past them, the radix sort's tiles of 2,048 keys (up to 131,072 keys) and of 4,096, its 64 count groups
+first size past them, the radix sort's tiles of 2,048 keys (up to 262,144 keys) and of 4,096, its 64 count groups
 and the launch that adds counts up (beyond 128 tiles), the run outputs' tiles
 of 4,096 positions and 64 of them looked back over at a time; with keys whose
 digits pile up in one bin, all equal (one run over every tile), descending, or
@@ -79,7 +79,7 @@ def test_dedup_equals_numpy(kind, n):
 
 
 @pytest.mark.parametrize("kind", ["table", "wide", "hot"])
-@pytest.mark.parametrize("n", [4097, 6143, 6144, 6145, 8191, 131072 - 2048, 131071, 131072, 131073, 135169])
+@pytest.mark.parametrize("n", [4097, 6143, 6144, 6145, 8191, 131072, 131073, 262144 - 2048, 262143, 262144, 262145, 266241])
 def test_two_round_tiles(kind, n):
     test_dedup_equals_numpy(kind, n)
 
@@ -87,7 +87,7 @@ def test_two_round_tiles(kind, n):
 def test_workspace_of_more_keys_serves_fewer():
     """A workspace sized for n keys is taken for every smaller batch, also across a change of tile size."""
     need, last = ctypes.c_uint64(), 0
-    for n in [1, 4096, 4097, 8192, 131071, 131072, 131073, 131200, 140000, 262144, 300000]:
+    for n in [1, 4096, 4097, 8192, 131072, 262143, 262144, 262145, 262200, 280000, 524288, 600000]:
         _lib.call("nve_amd_dedup_workspace_size", n, ctypes.byref(need))
         assert need.value >= last, n
         last = need.value
