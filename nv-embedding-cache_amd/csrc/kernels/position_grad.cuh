@@ -17,7 +17,13 @@ namespace nve_amd {
 // search that reads an offset per thread and step; the bags that start inside
 // the tile mark their first positions, and a running maximum spreads the marks.  (A
 // search per position is bound by its loads: 9.5 us for 262,144 positions of
-// 256 bags, with eight offsets a step 20 us; this takes 4.)
+// 256 bags, with eight offsets a step 20 us; this takes 4.)  A thread marks at most
+// kMarkSteps bags, each step a load's latency (0.9 us): where more bags start in the
+// tile (mostly empty ones), every position searches for its own.
+// Backprop of 2,000 keys in 1,000,000 bags, marking all of them and searching:
+// 861 and 57 us; in 65,536 bags 84 and 53; 262,144 keys in 4,000,000 bags 133 and
+// 131; at or below 16 steps a thread the marks are as fast or faster.
+constexpr int kMarkSteps = 16;
 template <int NT, int TILE>
 __device__ __forceinline__ void tile_rows(const PositionGrad& g, int64_t base, uint32_t* rows) {
   constexpr int kPer = TILE / NT;
@@ -46,12 +52,28 @@ __device__ __forceinline__ void tile_rows(const PositionGrad& g, int64_t base, u
   }
   __syncthreads();
   const int64_t first = lo;
+  const int64_t end = g.num_bags > 0 ? load_key(g.offsets, g.key_bytes, g.num_bags) - base : 0;
+  const int64_t past = first + (int64_t)kMarkSteps * NT;  // the first bag that no thread would mark
+  if (past < g.num_bags && load_key(g.offsets, g.key_bytes, past) - base < TILE) {  // uniform
+    uint32_t n[kPer];  // bags that start at or before the position, at least `first`
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) n[q] = lo;
+    for (uint32_t half, len = (uint32_t)g.num_bags - lo; len > 0; len -= half) {
+      half = (len + 1) / 2;
+#pragma unroll
+      for (int q = 0; q < kPer; ++q)
+        if (load_key(g.offsets, g.key_bytes, (int64_t)n[q] + half - 1) <= base + q * NT + tid) n[q] += half;
+    }
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) rows[q * NT + tid] = n[q] != 0 && q * NT + tid < end ? n[q] - 1u : kNoGradRow;
+    __syncthreads();
+    return;
+  }
   for (int64_t b = first + tid; b < g.num_bags; b += NT) {
     const int64_t x = load_key(g.offsets, g.key_bytes, b) - base;
     if (x >= TILE || x < 0) break;  // non-decreasing offsets: none of the later ones either
     atomicMax(&rows[x], (uint32_t)b + 1u);
   }
-  const int64_t end = g.num_bags > 0 ? load_key(g.offsets, g.key_bytes, g.num_bags) - base : 0;
   __syncthreads();
   uint32_t v[kPer], m = 0;
 #pragma unroll

@@ -1,8 +1,8 @@
 """Training backprop where the bag of every key position is found anew: batches
 of one workgroup and of several 4,096-key tiles, one bag to more bags than keys,
 bags that end at a tile's edge or span tiles, empty bags at either end,
-positions before the first bag and after the last one, and keys that need the
-sort on their exact bits.  Against the oracle, bit for bit."""
+positions before the first bag and after the last one, more bags in a tile than
+its threads mark (16 each), and keys that need the sort on their exact bits.  Against the oracle, bit for bit."""
 import numpy as np
 import pytest
 
@@ -23,6 +23,14 @@ def offsets_of(kind, n, rng):
     elif kind == "many":  # more bags than keys, most of them empty
         cut = np.sort(rng.integers(0, n + 1, size=2 * n + 3))
         cut[0], cut[-1] = 0, n
+    elif kind == "marked":  # as many bags as are marked start at the last key
+        cut = [0] + [n - 1] * (16 * 1024) + [n]
+    elif kind == "searched":  # and one more
+        cut = [0] + [n - 1] * (16 * 1024 + 1) + [n]
+    elif kind == "sparse":  # many times more bags than keys, some keys outside them
+        cut = np.sort(rng.integers(3, n - 2, size=70001))
+    elif kind == "front":  # a key in each of the first bags, all others empty
+        cut = np.concatenate([np.arange(n), np.full(50000, n)])
     elif kind == "outside":  # keys before the first bag and after the last
         cut = np.sort(rng.integers(n // 5, n - n // 5 + 1, size=70))
     else:  # 64 and 1,024 are the widths of a search step
@@ -34,7 +42,8 @@ def offsets_of(kind, n, rng):
 
 
 @pytest.mark.parametrize("pooling", [O.SUM, O.MEAN, O.WSUM, O.WMEAN])
-@pytest.mark.parametrize("kind", ["one", "edges", "many", "outside", "63", "64", "65", "1023", "1024", "1025"])
+@pytest.mark.parametrize("kind", ["one", "edges", "many", "outside", "63", "64", "65", "1023", "1024", "1025",
+                                  "marked", "searched", "sparse", "front"])
 @pytest.mark.parametrize("n,wide", [(900, False), (TILE, False), (TILE + 1, False), (3 * TILE + 50, False),
                                     (2 * TILE + 7, True)])
 def test_rows_of_every_position(n, wide, kind, pooling):
