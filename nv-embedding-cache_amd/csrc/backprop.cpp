@@ -124,6 +124,7 @@ int64_t pooling_backprop_run(int key_bytes, int64_t n, const void* keys, int poo
     NVE_HIP(launch_bag_denom(csr, key_bytes, num_bags, hotness, weights, wdt, mode == kBackpropWMean,
                              b.denom, s));
   const PositionGrad pg{mode, csr, key_bytes, num_bags, hotness, weights, wdt, b.denom, b.rows, b.nw, b.by_key};
+  PendingHead head(s);
   dedup_run(key_bytes, n, keys, unique_out, b.counts, nullptr, b.doff, b.dedup_ws, b.dedup_bytes, s,
             b.kidx, true, exact, &pg);
 
@@ -145,7 +146,7 @@ int64_t pooling_backprop_run(int key_bytes, int64_t n, const void* keys, int poo
   const int weighted = (mode == kBackpropWSum || mode == kBackpropMean || mode == kBackpropWMean) ? 1 : 0;
   NVE_HIP(launch_piece_pool(a, f16, weighted, s));
   NVE_HIP(launch_piece_combine(a, f16, s));
-  const DedupHead h = dedup_head(s);
+  const DedupHead h = head.read();
   if (!exact && dedup_spec_failed(h))  // keys differ above the speculated sort bits: all again, exactly
     return pooling_backprop_run(key_bytes, n, keys, pooling, sparse, offsets, num_bags, hotness, weights, wdt,
                                 grads_in, gdt, dim, unique_out, grads_out, ws, ws_bytes, s, true);

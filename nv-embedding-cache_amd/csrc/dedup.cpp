@@ -77,7 +77,7 @@ size_t dedup_workspace_bytes(int64_t n) {
 
 DedupHead dedup_head(hipStream_t s) {
   NVE_HIP(hipStreamSynchronize(s));
-  return *static_cast<DedupHead*>(pinned_slot());
+  return *static_cast<DedupHead*>(pinned_slot(kDedupHeadSlot));
 }
 
 int64_t dedup_run(int key_bytes, int64_t n, const void* keys, void* unique, void* counts,
@@ -89,7 +89,7 @@ int64_t dedup_run(int key_bytes, int64_t n, const void* keys, void* unique, void
   DedupBufs b = carve(ws, n);
   const DedupOut out{key_bytes, unique,  counts,
                      inverse,   offsets, pos_key,
-                     b.head,    static_cast<DedupHead*>(pinned_slot()), pg != nullptr ? *pg : PositionGrad{}};
+                     b.head,    static_cast<DedupHead*>(pinned_slot(kDedupHeadSlot)), pg != nullptr ? *pg : PositionGrad{}};
   if (n <= kSmallDedupKeys) {
     NVE_HIP(launch_dedup_small(keys, n, out, s));
   } else {

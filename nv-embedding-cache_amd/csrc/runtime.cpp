@@ -12,16 +12,16 @@
 
 namespace nve_amd {
 
-void* pinned_slot() {
-  // one pinned slot per thread, kept for the thread's life
-  thread_local void* slot = nullptr;
-  if (slot == nullptr) NVE_HIP(hipHostMalloc(&slot, kPinnedSlotBytes, hipHostMallocDefault));
-  return slot;
+void* pinned_slot(PinnedSlot use) {
+  // allocated once per thread, kept for the thread's life
+  thread_local void* slots = nullptr;
+  if (slots == nullptr) NVE_HIP(hipHostMalloc(&slots, kPinnedSlots * kPinnedSlotBytes, hipHostMallocDefault));
+  return static_cast<uint8_t*>(slots) + use * kPinnedSlotBytes;
 }
 
 void read_small(void* host, const void* dev, size_t bytes, hipStream_t stream) {
   NVE_CHECK(bytes <= kPinnedSlotBytes, "read_small reads at most 64 bytes");
-  void* slot = pinned_slot();
+  void* slot = pinned_slot(kReadSlot);
   NVE_HIP(launch_small_read(slot, dev, (int)bytes, stream));
   NVE_HIP(hipStreamSynchronize(stream));
   std::memcpy(host, slot, bytes);

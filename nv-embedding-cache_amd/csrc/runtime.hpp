@@ -226,10 +226,13 @@ const void* device_input(ExecutionContext& ctx, const char* name, const void* p,
 const void* host_input(ExecutionContext& ctx, const char* name, const void* p, size_t bytes,
                        hipStream_t stream);
 
-// The calling thread's pinned host memory (kPinnedSlotBytes), which kernels may
-// write results to that the thread reads after waiting for their stream.
+// Pinned host memory of the calling thread (kPinnedSlotBytes a slot), which
+// kernels may write results to that the thread reads after waiting for their
+// stream.  Each use has a slot of its own: a dedup's head is written while the
+// thread may already wait for something else.
+enum PinnedSlot { kReadSlot, kDedupHeadSlot, kPinnedSlots };
 constexpr size_t kPinnedSlotBytes = 64;
-void* pinned_slot();
+void* pinned_slot(PinnedSlot use);
 
 // Copies `bytes` (at most 64) of device memory to `host` and waits for
 // `stream`.  The copy lands in a pinned per-thread slot first: a pageable
