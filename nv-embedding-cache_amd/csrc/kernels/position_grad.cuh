@@ -18,12 +18,12 @@ namespace nve_amd {
 // the tile mark their first positions, and a running maximum spreads the marks.  (A
 // search per position is bound by its loads: 9.5 us for 262,144 positions of
 // 256 bags, with eight offsets a step 20 us; this takes 4.)  A thread marks at most
-// kMarkSteps bags, each step a load's latency (0.9 us): where more bags start in the
-// tile (mostly empty ones), every position searches for its own.
-// Backprop of 2,000 keys in 1,000,000 bags, marking all of them and searching:
-// 861 and 57 us; in 65,536 bags 84 and 53; 262,144 keys in 4,000,000 bags 133 and
-// 131; at or below 16 steps a thread the marks are as fast or faster.
-constexpr int kMarkSteps = 16;
+// kMarkSteps bags, each step a load's latency (0.8 us): where more bags start in the
+// tile (mostly empty ones), every position searches for its own.  The line is
+// where the two meet: backprop of 2,000 keys with 4,096, 8,192 and 16,384 bags in a
+// tile takes 46.5, 50 and 57 us with marks and 49 with the search, of 100,000 keys 83,
+// 86 and 93 us and 81-82.  (All bags marked, 2,000 keys in 1,000,000 bags: 861 us; 57 now.)
+constexpr int kMarkSteps = 8;
 template <int NT, int TILE>
 __device__ __forceinline__ void tile_rows(const PositionGrad& g, int64_t base, uint32_t* rows) {
   constexpr int kPer = TILE / NT;

@@ -2,7 +2,8 @@
 of one workgroup and of several 4,096-key tiles, one bag to more bags than keys,
 bags that end at a tile's edge or span tiles, empty bags at either end,
 positions before the first bag and after the last one, more bags in a tile than
-its threads mark (16 each), and keys that need the sort on their exact bits.  Against the oracle, bit for bit."""
+its threads mark (8 each), and keys that need the sort on their exact bits.
+Against the oracle, bit for bit."""
 import numpy as np
 import pytest
 
@@ -24,9 +25,9 @@ def offsets_of(kind, n, rng):
         cut = np.sort(rng.integers(0, n + 1, size=2 * n + 3))
         cut[0], cut[-1] = 0, n
     elif kind == "marked":  # as many bags as are marked start at the last key
-        cut = [0] + [n - 1] * (16 * 1024) + [n]
+        cut = [0] + [n - 1] * (8 * 1024) + [n]
     elif kind == "searched":  # and one more
-        cut = [0] + [n - 1] * (16 * 1024 + 1) + [n]
+        cut = [0] + [n - 1] * (8 * 1024 + 1) + [n]
     elif kind == "sparse":  # many times more bags than keys, some keys outside them
         cut = np.sort(rng.integers(3, n - 2, size=70001))
     elif kind == "front":  # a key in each of the first bags, all others empty
