@@ -372,6 +372,45 @@ __device__ __forceinline__ Slice lane_slice(uint32_t value_bytes, int gl, uint32
   return s;
 }
 
+// part[q] = the keys that row q of each G-lane group resolved (G a multiple of
+// 16), in every row of the group.
+template <int G>
+__device__ __forceinline__ void spread_rows(uint32_t v, uint32_t (&part)[G / 16]) {
+  if constexpr (G == 64) {
+    const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const auto r = __builtin_amdgcn_permlane16_swap(h[q], h[q], false, false);
+      part[2 * q] = r[0];
+      part[2 * q + 1] = r[1];
+    }
+  } else if constexpr (G == 32) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    part[0] = r[0];
+    part[1] = r[1];
+  } else {
+    part[0] = v;
+  }
+}
+template <int G, bool W>
+__device__ __forceinline__ void spread_keys(const LaneKey& k, LaneKey (&part)[G / 16]) {
+  uint32_t lo[G / 16], hi[G / 16], w[G / 16], ws[G / 16];
+  spread_rows<G>((uint32_t)k.addr, lo);
+  spread_rows<G>((uint32_t)(k.addr >> 32), hi);
+  if constexpr (W) {
+    spread_rows<G>(__float_as_uint(k.w), w);
+    spread_rows<G>(__float_as_uint(k.ws), ws);
+  }
+#pragma unroll
+  for (int q = 0; q < G / 16; ++q) {
+    part[q] = LaneKey{((uint64_t)hi[q] << 32) | lo[q], 0.0f, 0.0f, Meta{0.0f, 0.0f}};
+    if constexpr (W) {
+      part[q].w = __uint_as_float(w[q]);
+      part[q].ws = __uint_as_float(ws[q]);
+    }
+  }
+}
+
 template <int SDT, int VB, int G, bool W, bool CACHE = false>
 __global__ __launch_bounds__(1024) void pool_split_kernel(
     std::conditional_t<CACHE, SplitCacheArgs, SplitArgs> a) {
@@ -381,7 +420,14 @@ __global__ __launch_bounds__(1024) void pool_split_kernel(
   // rows in flight: fewer with 16 values a lane or weights and a cache, whose
   // batch would leave the registers of a 1024-thread workgroup
   constexpr int UMAX = E > 8 || (W && CACHE) ? 8 : 16;
-  constexpr int U = K < UMAX ? K : UMAX;  // a round's keys in K / U batches
+  constexpr int U = K < UMAX ? K : UMAX;  // a round's keys in batches of U
+  // A probe of the cache's tags costs far more than the moves of its result: the
+  // lanes of a wide group probe a key each, and the rows' results are spread
+  // over the group 16 at a time.  256 bags of ~1,000 keys, every row of the group
+  // probing the same 16 keys and this, all hits: 512-byte rows 15.1 and 13.9 us,
+  // 1,024-byte fp32 rows 22.9 and 19.2, 2,400-byte rows 62.3 and 51.0; 4,096 bags of
+  // ~40 keys, 512-byte fp32 rows 11.8 and 10.5 us.
+  constexpr int R = CACHE ? G : K;  // keys of a round
   extern __shared__ float lds[];
 
   const int tid = threadIdx.x;
@@ -421,20 +467,20 @@ __global__ __launch_bounds__(1024) void pool_split_kernel(
   float wsum = 0.0f;
 
   uint32_t misses = 0;
-  const int kl = gl & (K - 1);
-  // one key per lane and round of K keys, loaded a round ahead
+  const int kl = gl & (R - 1);
+  // one key per lane and round of R keys, loaded a round ahead
   int64_t ahead = cs + kl < ce ? load_key(a.keys, a.key_bytes, cs + kl) : -1;
-  for (int64_t k0 = cs; k0 < ce; k0 += K) {
+  for (int64_t k0 = cs; k0 < ce; k0 += R) {
     const int64_t kk = k0 + kl;
     const int64_t key = ahead;
-    if (kk + K < ce) ahead = load_key(a.keys, a.key_bytes, kk + K);
+    if (kk + R < ce) ahead = load_key(a.keys, a.key_bytes, kk + R);
     LaneKey lk{(uint64_t)g_zero_row, 0.0f, 0.0f, Meta{0.0f, 0.0f}};
     if (kk < ce) {
       bool real;
       if constexpr (CACHE) {
         bool miss;
         const uint64_t row = cache_row(a, key, &miss);
-        misses += miss && gl < K ? 1u : 0u;
+        misses += miss ? 1u : 0u;
         real = row != 0;
         if (real) lk.addr = row;
       } else {
@@ -449,14 +495,17 @@ __global__ __launch_bounds__(1024) void pool_split_kernel(
         lk.w = real ? lk.ws : 0.0f;
       }
     }
-    const int n = (int)((ce - k0) < K ? (ce - k0) : K);
+    const int n = (int)((ce - k0) < R ? (ce - k0) : R);
+    LaneKey part[R / K];
+    if constexpr (R > K) spread_keys<R, W>(lk, part);
+    else part[0] = lk;
     // batch from key j0 of the round on (compile time, so every lane move has
     // an immediate source lane)
     auto batch = [&](auto jc) {
       constexpr int j0 = decltype(jc)::value;
-      if (j0 < n) add_batch<SDT, VB, K, U, W, j0>(lk, sl.off, acc, wsum);
+      if (j0 < n) add_batch<SDT, VB, K, U, W, j0 % K>(part[j0 / K], sl.off, acc, wsum);
     };
-    for_batches<U, 0, K / U>(batch);
+    for_batches<U, 0, R / U>(batch);
   }
 
   // butterfly over the wave's groups (the same pairing and additions as pool_kernel)

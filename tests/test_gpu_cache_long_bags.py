@@ -17,7 +17,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from nve_helpers import float_table, rel_close, stream_ptr, to_dev, vp
+from nve_helpers import float_table, pooled_f16_close, rel_close, stream_ptr, to_dev, vp
 from oracle import oracle as O
 from pynve import _lib
 from test_gpu_cache_lookup import CachedTable
@@ -122,4 +122,44 @@ def test_hit_miss_decisions_against_the_cache_model(lens):
     assert rel_close(got, ref.reshape(bags, dim), 1e-5)
     assert np.all(got[5] == 0)
     assert abs(hr - (1.0 - misses / n)) < 1e-6
+    close(layer, lctx, ct)
+
+
+# widths of 4-, 8- and 16-byte slices, whole and overlapping, in lane groups of 8 to 64 and in one to five columns
+LAYOUTS = [(O.F16, d) for d in (16, 17, 33, 64, 100, 136, 256, 264, 512, 513, 1024, 1200)] + \
+          [(O.F32, d) for d in (8, 9, 16, 32, 50, 64, 128, 132, 256, 257, 600, 1024)]
+
+
+@pytest.mark.parametrize("lens", [(33, 64, 30), (64, 140, 20), (300, 1100, 9)], ids=["wave", "two", "long"])
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("dtype,dim", LAYOUTS)
+def test_every_slice_layout(dtype, dim, weighted, lens):
+    """Cached values negated, as above: bags of one wave and of several, whose groups' chunks end inside a round of
+    8 to 64 keys; the sum and the exact miss count, which only the first column adds to."""
+    key_bytes = 4 if dim % 3 == 0 else 8
+    rng = np.random.default_rng(7 * dim + dtype + lens[0] + weighted)
+    es, kt = O.value_bytes(dtype), np.int64 if key_bytes == 8 else np.int32
+    rows, bags = 3000, lens[2]
+    tb = float_table(rng, rows, dim, dtype, dyadic_values=False)
+    ct = CachedTable(tb, 1200 * (dim * es + 300), key_bytes, value_dtype=DT[dtype])
+    ct.model.insert_keys(rng.choice(1200, size=1500).astype(kt), uvm=ct.uvm_np.reshape(-1))
+    ct.model.data().reshape(-1, es)[:, es - 1] ^= np.uint8(0x80)
+    ct.load_model()
+    cuts = rng.integers(lens[0], lens[1], size=bags)
+    cuts[:3] = [0, 1, lens[1]]
+    off = np.zeros(bags + 1, kt)
+    off[1:] = np.cumsum(cuts)
+    n = int(off[-1])
+    keys = np.where(rng.uniform(size=n) < 0.8, rng.integers(0, 1200, size=n), rng.integers(0, rows, size=n)).astype(kt)
+    w = rng.uniform(0, 1, size=n).astype(np.float32) if weighted else None
+    layer, lctx = layer_over(ct, key_bytes)
+    pooling = _lib.POOL_WMEAN if weighted else _lib.POOL_SUM
+    got, hr = pooled(layer, lctx, keys, dim, dtype, pooling, off, bags, 0, w)
+    rows_ptr, _, misses = ct.model.resolve(keys, ct.uvm_np.reshape(-1))
+    ref = O.pool(rows_ptr, dtype, dim, O.CSR, pooling, n, off, bags, 0, w, O.F32, dtype).reshape(bags, dim)
+    if dtype == O.F16:
+        assert pooled_f16_close(got, ref.view(np.uint16))
+    else:
+        assert rel_close(got, ref, 1e-5)
+    assert 0.0 < hr < 1.0 and abs(hr - (1.0 - misses / n)) < 1e-6
     close(layer, lctx, ct)
