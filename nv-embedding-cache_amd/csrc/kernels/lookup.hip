@@ -595,10 +595,10 @@ int pool_groups_per_bag(const PoolLaunch& a, int g) {
     gpb = pow2_ceil(a.force_split);
   } else if (a.force_split == 0) {
     // split long bags when there are too few bags to keep the chip's 256 CUs
-    // streaming: aim at ~16 keys per group, at least a whole wave per bag
+    // streaming: aim at ~16 keys per group
     if (avg > 32 && bags * (int64_t)g < 256LL * 1024) {
       const int64_t want = avg / 16;
-      while ((int64_t)gpb * 2 <= want || gpb * g < 64) gpb <<= 1;
+      while ((int64_t)gpb * 2 <= want) gpb <<= 1;
     }
   }
   return gpb * g > 1024 ? 1024 / g : gpb;
@@ -625,7 +625,24 @@ bool pool_geometry(const PoolLaunch& a, PoolGeometry* g) {
   const int passes = (int)((nv + G - 1) / G);
   const int64_t bags = a.num_bags;
   const int64_t avg = a.keys_per_bag > 0 ? a.keys_per_bag : (bags > 0 ? a.num_keys / bags : 0);
-  const int gpb = pool_groups_per_bag(a, G);
+  int gpb = pool_groups_per_bag(a, G);
+  if (gpb > 1 && a.force_split == 0) {
+    // A bag gets up to a whole wave while the split leaves fewer than three waves
+    // per SIMD (1,024 of them): rows of under 32 bytes take few lanes, and 16 keys a
+    // group are a long chain of loads.  Past that more waves only add butterflies
+    // and idle lanes.  Bags of ~35 keys, groups of 2 or 4 lanes cut at 16 keys a group,
+    // with this rule and at a whole wave: 24-byte fp16 rows, 1,024 bags 8.9, 4.8 and
+    // 4.8 us, 8,192 bags 9.3, 6.9 and 8.5, 32,000 bags 15.0, 15.0 and 25.1; 28-byte fp32
+    // rows (8 lanes), 4,096 bags 5.8, 5.1 and 5.1, 16,384 bags 8.1, 8.1 and 11.7.
+    // Groups of one lane walk the keys alone and gain from a wave up to 32,768 bags
+    // (8-byte rows, 1,024 bags 29 and 5 us, 16,384 bags 29 and 15, 32,000 bags of ~64
+    // keys 32 and 34, 65,536 bags of ~35 keys 41 and 51).
+    const int64_t wave = 64;
+    if (G == 1 && bags <= 32768)
+      gpb = gpb < wave ? (int)wave : gpb;
+    else
+      while (gpb * G < wave && bags * gpb * G < 3 * 1024 * wave) gpb <<= 1;
+  }
   int threads;
   if (gpb == 1) {
     threads = 256;

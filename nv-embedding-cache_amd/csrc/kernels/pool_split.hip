@@ -50,6 +50,7 @@ bool pool_slices(const PoolLaunch& a, PoolSlices* g) {
     while (g->g < slices && g->g < 64) g->g *= 2;
     g->columns = (int)((slices + g->g - 1) / g->g);
     g->gpb = pool_groups_per_bag(a, g->g);
+    if (a.force_split == 0 && g->gpb > 1 && g->gpb * g->g < 64) g->gpb = 64 / g->g;  // whole waves
   };
   cut(area > 64 ? 16 : area > 32 ? 8 : 4);
   // Bytes widen to 16 values a lane in a 16-byte slice: 8-byte slices halve the

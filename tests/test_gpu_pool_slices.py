@@ -131,3 +131,12 @@ def test_several_tables_of_bags_that_fill_no_workgroup(dtype, count, out):
         ref = oracle_pool(tables[t], keys[s:e], dtype, count, O.CSR, O.MEAN, off[t * bags:(t + 1) * bags + 1] - s, bags,
                           0, None, 0, out)
         assert np.array_equal(got[:, t], ref.view(bits))
+
+
+# rows under 32 bytes (the general kernel) in groups of 1, 2, 4, 8 and 16 lanes; numbers of bags on both sides of the
+# lines where such a bag's share of a wave changes
+@pytest.mark.parametrize("bags", [300, 3100, 6200, 12300, 33000])
+@pytest.mark.parametrize("dtype,count", [(O.F16, 4), (O.F16, 12), (O.F32, 4), (O.F32, 7), (O.QI8_F32, 8), (O.QU8_F32, 30)])
+def test_narrow_rows_in_bags_of_a_few_dozen_keys(dtype, count, bags):
+    lens = np.random.default_rng(bags).integers(20, 60, size=bags)
+    check(dtype, count, _lib.POOL_WMEAN if count % 8 else _lib.POOL_SUM, lens, 0, False, bags + count)
