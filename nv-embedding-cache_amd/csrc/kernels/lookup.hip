@@ -12,6 +12,8 @@
 // included) and their row addresses broadcast inside the group with
 // ds_bpermute; a batch's row loads are all issued before any is consumed.
 // The find-and-pool kernel lives in pool_kernel.cuh.
+#include <algorithm>
+
 #include "device_common.cuh"
 #include "lane_moves.cuh"
 #include "pool_launch.hpp"
@@ -630,18 +632,19 @@ bool pool_geometry(const PoolLaunch& a, PoolGeometry* g) {
     // A bag gets up to a whole wave while the split leaves fewer than three waves
     // per SIMD (1,024 of them): rows of under 32 bytes take few lanes, and 16 keys a
     // group are a long chain of loads.  Past that more waves only add butterflies
-    // and idle lanes.  Bags of ~35 keys, groups of 2 or 4 lanes cut at 16 keys a group,
-    // with this rule and at a whole wave: 24-byte fp16 rows, 1,024 bags 8.9, 4.8 and
-    // 4.8 us, 8,192 bags 9.3, 6.9 and 8.5, 32,000 bags 15.0, 15.0 and 25.1; 28-byte fp32
+    // and idle lanes.  Bags of ~35 keys cut at 16 keys a group, with this rule and at
+    // a whole wave: 24-byte fp16 rows (4 lanes), 1,024 bags 8.9, 4.8 and 4.8 us, 8,192 bags 9.3, 6.9 and 8.5, 32,000 bags 15.0, 15.0 and 25.1; 28-byte fp32
     // rows (8 lanes), 4,096 bags 5.8, 5.1 and 5.1, 16,384 bags 8.1, 8.1 and 11.7.
-    // Groups of one lane walk the keys alone and gain from a wave up to 32,768 bags
-    // (8-byte rows, 1,024 bags 29 and 5 us, 16,384 bags 29 and 15, 32,000 bags of ~64
-    // keys 32 and 34, 65,536 bags of ~35 keys 41 and 51).
+    // A group of one lane walks its keys alone and takes at most 4 of them at any
+    // number of bags, one of two lanes (with weights, of four) 20 instead of 31: cut at
+    // 16 keys a group, at a whole wave and so, 16-byte rows, 65,536 bags of ~35 keys 51,
+    // 60 and 39 us, 32,000 bags of ~100 weighted keys 82, 55 and 50; 12-byte int8 rows,
+    // 50,000 bags of ~50 keys 103, 85 and 91; 20-byte ones, 32,000 bags of ~100 weighted
+    // keys 66, 56 and 53.
     const int64_t wave = 64;
-    if (G == 1 && bags <= 32768)
-      gpb = gpb < wave ? (int)wave : gpb;
-    else
-      while (gpb * G < wave && bags * gpb * G < 3 * 1024 * wave) gpb <<= 1;
+    const int64_t most = G == 1 ? 4 : G == 2 || (G == 4 && a.weighted) ? 20 : 32;
+    while (gpb * G < wave && avg > most * gpb) gpb <<= 1;
+    while (gpb * G < wave && bags * gpb * G < 3 * 1024 * wave) gpb <<= 1;
   }
   int threads;
   if (gpb == 1) {
