@@ -140,3 +140,15 @@ def test_several_tables_of_bags_that_fill_no_workgroup(dtype, count, out):
 def test_narrow_rows_in_bags_of_a_few_dozen_keys(dtype, count, bags):
     lens = np.random.default_rng(bags).integers(20, 60, size=bags)
     check(dtype, count, _lib.POOL_WMEAN if count % 8 else _lib.POOL_SUM, lens, 0, False, bags + count)
+
+
+@pytest.mark.parametrize("dtype,count,bags,pooling,whole", [
+    (O.F16, 64, 16384, _lib.POOL_WSUM, True), (O.F16, 64, 16383, _lib.POOL_WSUM, False),
+    (O.F32, 64, 8192, _lib.POOL_SUM, True), (O.F32, 64, 8191, _lib.POOL_SUM, False),
+    (O.QI8_F32, 130, 8192, _lib.POOL_WMEAN, True), (O.F16, 256, 50, _lib.POOL_WMEAN, True),
+    (O.F16, 256, 50, _lib.POOL_MEAN, False), (O.F16, 256, 4096, _lib.POOL_MEAN, True)])
+def test_bags_of_a_few_dozen_keys(dtype, count, bags, pooling, whole):
+    """Bags of 33 to 64 keys on both sides of the lines where a wave shares a bag: one added by a single group equals
+    the oracle bit for bit, one that is cut stays within the tolerance of its order."""
+    lens = np.random.default_rng(bags).integers(25, 70, size=bags)
+    check(dtype, count, pooling, lens, 1, whole, bags + count)
