@@ -641,12 +641,11 @@ struct ShortArgsMT : ShortArgs {
   uint32_t table_rows[kMaxPoolTables];
 };
 
-template <int SDT, int VB, int G, bool W, bool MT, int UMAX>
+template <int SDT, int VB, int G, bool W, bool MT, int U>
 __global__ __launch_bounds__(256) void pool_short_kernel(std::conditional_t<MT, ShortArgsMT, ShortArgs> a) {
   constexpr int ES = Fmt<SDT>::esize;
   constexpr int E = VB / ES;
   constexpr int K = kRound<G>;
-  constexpr int U = K < UMAX ? K : UMAX;
 
   const int tid = threadIdx.x;
   const int gl = tid & (G - 1);
@@ -806,11 +805,11 @@ hipError_t launch_short_g(const PoolLaunch& a, const PoolSlices& g, hipStream_t 
   // registers of 8 or 16 rows would keep waves out (26 tables of 8,192 bags of
   // ~20 keys: 4 -> 104 us, 8 -> 111 us).  Launches of at most 4 waves per SIMD
   // lose none to 8 rows (16,384 bags of ~30 200-byte rows: 13.9 -> 13.6 us),
-  // and bags past 48 keys keep 16 (8 where a lane decodes 16 values).
+  // and bags past 48 keys keep 16 (8 where a lane decodes 16 values or a round has 8 keys).
   const int64_t avg = a.keys_per_bag > 0 ? a.keys_per_bag
                                          : a.num_keys / (a.num_bags > 0 ? a.num_bags : 1);
   const bool few = (int64_t)grid.x * grid.y * grid.z <= 4 * 256;  // workgroups of a wave per SIMD
-  constexpr int kWide = VB / Fmt<SDT>::esize > 8 ? 8 : 16;
+  constexpr int kWide = VB / Fmt<SDT>::esize > 8 || kRound<G> < 16 ? 8 : 16;
 #define NVE_LAUNCH_SHORT(W, U) \
   hipLaunchKernelGGL((pool_short_kernel<SDT, VB, G, W, MT, U>), grid, block, 0, stream, s)
   if (avg > 48) {
@@ -825,29 +824,46 @@ hipError_t launch_short_g(const PoolLaunch& a, const PoolSlices& g, hipStream_t 
 }
 
 // MT launches take f16 / f32 rows only.
-template <int SDT, int VB, int G>
+template <int SDT, int VB, int G, bool SHORT = true, bool SPLIT = true>
 hipError_t launch_slices_g(const PoolLaunch& a, const PoolSlices& g, hipStream_t stream) {
-  if (g.gpb > 1) return launch_split_g<SDT, VB, G>(a, g, stream);
-  if constexpr (Fmt<SDT>::meta == 0) {
-    if (a.num_tables > 0) return launch_short_g<SDT, VB, G, true>(a, g, stream);
+  if constexpr (SPLIT) {
+    if (g.gpb > 1) return launch_split_g<SDT, VB, G>(a, g, stream);
   }
-  return launch_short_g<SDT, VB, G, false>(a, g, stream);
+  if constexpr (SHORT) {
+    if constexpr (Fmt<SDT>::meta == 0) {
+      if (a.num_tables > 0) return launch_short_g<SDT, VB, G, true>(a, g, stream);
+    }
+    if (g.gpb == 1) return launch_short_g<SDT, VB, G, false>(a, g, stream);
+  }
+  return hipErrorInvalidValue;
 }
 
+// The slices that pool_slices chooses: 16 bytes for wide f16 / f32 rows, for wide
+// byte rows 8 bytes up to 128 of them and, where a group has a bag to itself, up to
+// 512, else 16.
 template <int SDT>
 hipError_t launch_slices_sdt(const PoolLaunch& a, const PoolSlices& g, hipStream_t stream) {
   switch (g.vb * 100 + g.g) {
     case 408: return launch_slices_g<SDT, 4, 8>(a, g, stream);
     case 808: return launch_slices_g<SDT, 8, 8>(a, g, stream);
-    case 816: return launch_slices_g<SDT, 8, 16>(a, g, stream);
-    case 832: return launch_slices_g<SDT, 8, 32>(a, g, stream);
-    case 864: return launch_slices_g<SDT, 8, 64>(a, g, stream);
-    case 1608: return launch_slices_g<SDT, 16, 8>(a, g, stream);
-    case 1616: return launch_slices_g<SDT, 16, 16>(a, g, stream);
-    case 1632: return launch_slices_g<SDT, 16, 32>(a, g, stream);
     case 1664: return launch_slices_g<SDT, 16, 64>(a, g, stream);
-    default: return hipErrorInvalidValue;
   }
+  if constexpr (Fmt<SDT>::esize == 1) {
+    switch (g.vb * 100 + g.g) {
+      case 816: return launch_slices_g<SDT, 8, 16>(a, g, stream);
+      case 832: return launch_slices_g<SDT, 8, 32, true, false>(a, g, stream);
+      case 864: return launch_slices_g<SDT, 8, 64, true, false>(a, g, stream);
+      case 1616: return launch_slices_g<SDT, 16, 16, false, true>(a, g, stream);
+      case 1632: return launch_slices_g<SDT, 16, 32, false, true>(a, g, stream);
+    }
+  } else {
+    switch (g.vb * 100 + g.g) {
+      case 1608: return launch_slices_g<SDT, 16, 8>(a, g, stream);
+      case 1616: return launch_slices_g<SDT, 16, 16>(a, g, stream);
+      case 1632: return launch_slices_g<SDT, 16, 32>(a, g, stream);
+    }
+  }
+  return hipErrorInvalidValue;
 }
 
 }  // namespace
