@@ -22,11 +22,12 @@ CDT = {O.F32: _lib.DT_F32, O.F16: _lib.DT_F16, O.QI8_F32: _lib.DT_QI8_F32, O.QI8
 GUARD = 64
 
 # (type, values per row): 31 / 32 / 33 bytes and 64 / 65, 128 / 129 (slice widths), 8 to 64 slices and one more
-# (lane groups, columns), 4,096 bytes (the widest row of these kernels) and wider
+# (lane groups, columns), 4,096 bytes (the widest row of these kernels) and wider; of the byte rows past 512 those of
+# whole 16-byte slices, whose 16 values a lane are stored through LDS, the second column's too
 FLOATS = [(O.F16, d) for d in (15, 16, 17, 32, 33, 63, 65, 100, 129, 256, 512, 513, 2048, 2050)] + \
          [(O.F32, d) for d in (7, 8, 9, 16, 17, 31, 50, 65, 128, 255, 257, 600, 1024, 1025)]
 QUANT = [(t, d) for t in (O.QI8_F32, O.QI8_F16, O.QU8_F32, O.QU8_F16, O.XI8A_F32, O.XE4M3_F32)
-         for d in (30, 34, 66, 128, 136, 514, 1030)]
+         for d in (30, 32, 34, 66, 128, 136, 300, 512, 514, 528, 1030, 2048)]
 
 
 def pooled(tb, dtype, count, keys, pooling, off, w, out_dtype, shift):
@@ -51,12 +52,13 @@ def pooled(tb, dtype, count, keys, pooling, off, w, out_dtype, shift):
     return raw[start:start + nb].view(np.uint16 if out_dtype == O.F16 else np.float32).reshape(bags, count)
 
 
-def check(dtype, count, pooling, lens, shift, exact, seed):
+def check(dtype, count, pooling, lens, shift, exact, seed, out_dtype=None):
     rng = np.random.default_rng(seed)
     rows = 3000
     quant = O.meta_bytes(dtype) > 0
     tb = quant_table(rng, rows, count, dtype) if quant else float_table(rng, rows, count, dtype, dyadic_values=False)
-    out_dtype = dtype if not quant else O.F16 if dtype in (O.QI8_F16, O.QU8_F16) else O.F32
+    if out_dtype is None:
+        out_dtype = dtype if not quant else O.F16 if dtype in (O.QI8_F16, O.QU8_F16) else O.F32
     off = np.zeros(len(lens) + 1, np.int64)
     off[1:] = np.cumsum(lens)
     keys = rng.integers(0, rows, size=int(off[-1])).astype(np.int64)
@@ -92,6 +94,14 @@ def test_short_bags_equal_the_oracle_bitwise(dtype, count, pooling, shift):
     check(dtype, count, pooling, lens, shift, True, 31 * count + pooling)
 
 
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("dtype", [O.XI8A_F32, O.XE4M3_F32])
+@pytest.mark.parametrize("count", [34, 136, 300, 528, 1024, 1030, 2048])
+def test_fp32_scaled_bytes_to_fp16(dtype, count, shift):
+    lens = np.diff(csr_offsets(np.random.default_rng(count), 70, 40))
+    check(dtype, count, _lib.POOL_WMEAN, lens, shift, True, count, O.F16)
+
+
 @pytest.mark.parametrize("pooling", [_lib.POOL_MEAN, _lib.POOL_WMEAN])
 @pytest.mark.parametrize("dtype,count", FLOATS + QUANT)
 def test_long_bags_within_tolerance(dtype, count, pooling):
@@ -100,7 +110,8 @@ def test_long_bags_within_tolerance(dtype, count, pooling):
 
 
 @pytest.mark.parametrize("out", [O.F16, O.F32])
-@pytest.mark.parametrize("dtype,count", [(O.F16, 100), (O.F16, 128), (O.F32, 36), (O.F16, 33)])
+@pytest.mark.parametrize("dtype,count", [(O.F16, 100), (O.F16, 128), (O.F32, 36), (O.F16, 33), (O.F16, 520),
+                                         (O.F16, 1024), (O.F32, 300)])
 def test_several_tables_of_bags_that_fill_no_workgroup(dtype, count, out):
     """Bags per table that are no multiple of a workgroup's, tables at odd offsets: each output column bitwise."""
     rng = np.random.default_rng(count)
