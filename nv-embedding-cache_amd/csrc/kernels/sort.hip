@@ -26,15 +26,19 @@
 // published word holds count and state together (one 64-bit store), so no other
 // memory has to be ordered against it.
 //
-// Bound: latency (a pass moves 24 bytes a key, 6 MB at 262,144 keys).  Three
-// launches per pass (tile counts, a scan of each digit's row, the scatter) took
-// nine launches for the three passes of a table's keys; the four of this sort and
-// the one launch of the dedup's runs take the dedup of 8,192 keys from 67 to 44 us,
-// of 32,768 keys from 66 to 51, of 131,072 keys from 67 to 61, of 262,144 keys from 73 to 71
-// and of 1,000,000 keys from 122 to 108.  Tiles are large so that each has few
-// predecessors: with 1024-key tiles every one of 256 tiles walks back through most
-// of them.  Nor do more words per step of the walk help (4,096-key tiles, 1,000,000 keys:
-// kLookAhead 4, 8, 16 and 32 take 107.6, 109.5, 112 and 118 us): the walk is bound
+// Bound: latency.  A pass moves 24 bytes a key (6 MB at 262,144 keys), and each of its
+// tiles also reads the digit counts of up to 64 counting workgroups (128 KB from L2:
+// 8 MB for the 64 tiles of 262,144 keys).  Three launches per pass (tile counts, a
+// scan of each digit's row, the scatter) took nine launches for the three passes of
+// a table's keys; the four of this sort and the one launch of the dedup's runs take
+// the dedup of 8,192 keys from 70 to 45 us, of 32,768 keys from 71 to 51, of 131,072
+// keys from 70 to 61, of 262,144 keys from 74 to 71 and of 1,000,000 keys from 123 to
+// 107.  Keys that differ in all 64 bits take eight passes over 450,000 to 600,000 keys
+// 2 to 4 % longer than the three launches each did (304 and 316 us for 600,000), one
+// key repeated 4,000,000 times 5 % (267 and 281); of 1,000,000 such keys 407 and 353 us.
+// Tiles are large so that each has few predecessors: with 1024-key tiles every one of
+// 256 tiles walks back through most of them.  Nor do more words per step of the walk
+// help (1,000,000 keys: kLookAhead 4 and 8 take 107.5 and 109.7 us): the walk is bound
 // by the words it reads.
 //
 // The exclusive scan of an array (run heads in the insert) is
@@ -425,12 +429,15 @@ size_t scan_temp_bytes(int64_t m) {
 namespace {
 // Rounds of 64 keys per wave, and so the tile of a sweep (1,024 keys per round).
 // Two rounds halve a tile's chain of ranking rounds and double the workgroups
-// where 4,096-key tiles leave most CUs idle, but past 128 tiles a tile walks back
-// over too many others.  Dedup with two and with four rounds (8 words per step of the
-// walk): 8,192 keys 44.4 and 51.0 us, 32,768 keys 50.8 and 56.5, 131,072 keys 61.6
-// and 64.4, 262,144 keys 72.2 and 73.2, 1,000,000 keys 127 and 109.  (One round up to
-// 16,384 keys: within 0.3 us of two at 8,192 and 16,384 keys, 1.4 us less at 5,000.)
-constexpr int64_t kTwoRoundKeys = 262144;
+// where 4,096-key tiles leave most CUs idle, but a tile walks back over twice as many
+// others, and every tile adds up the counting workgroups' parts.  Dedup with two and
+// with four rounds: 8,192 keys 45.1 and 51.0 us, 32,768 keys 51.0 and 56.8, 131,072
+// keys 61.2 and 64.9, 200,000 keys 67.4 and 68.2, 262,144 keys 71.4 and 71.2 (a backprop
+// of them 121.7 and 119.2), 300,000 keys 78.6 and 77.1, 400,000 keys 84.5 and 81.8,
+// 1,000,000 keys 126.4 and 107.5: the line lies between 200,000 and 262,144, at 112
+// tiles.  (One round up to 16,384 keys: within 0.3 us of two at 8,192 and 16,384 keys,
+// 1.4 us less at 5,000.)
+constexpr int64_t kTwoRoundKeys = 112 * 2048;
 int tile_items(int64_t n) { return n <= kTwoRoundKeys ? 2 : 4; }
 int64_t tiles_of(int64_t n) {
   const int64_t tile = kTileThreads * tile_items(n);
@@ -439,8 +446,11 @@ int64_t tiles_of(int64_t n) {
 // The most tiles of any batch of at most n keys: storage sized for n serves them all.
 int64_t most_tiles(int64_t n) { return std::max(tiles_of(n), tiles_of(std::min(n, kTwoRoundKeys))); }
 int64_t pass_words(int64_t tiles) { return 1 + tiles * kMaxBins; }
-// past this many tiles one launch adds the counts up
-constexpr int64_t kMaxAddingTiles = 128;
+// Past this many tiles (more than run at once, one on each CU) one launch adds the
+// counts up.  With it and without: backprop of 600,000 keys (147 tiles) 149.9 and 146.2
+// us, dedup of 700,000 keys 97.8 and 96.6, of 1,100,000 keys (269 tiles) 133.4 and
+// 136.3, of 4,000,000 keys 292 and 300.
+constexpr int64_t kMaxAddingTiles = 256;
 }  // namespace
 
 int64_t radix_span_parts(int64_t n) {

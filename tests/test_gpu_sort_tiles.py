@@ -1,8 +1,9 @@
 """The sorted dedup at the sizes where its work is cut anew: the single
 workgroup's 1 and 4 keys per thread (1,024 and 4,096 keys) and the
-first size past them, the radix sort's tiles of 2,048 keys (up to 262,144 keys) and of 4,096, its 64 count groups
-and the launch that adds counts up (beyond 128 tiles), the run outputs' tiles
-of 4,096 positions and 64 of them looked back over at a time; with keys whose
+first size past them, the radix sort's tiles of 2,048 keys (up to 229,376 keys) and
+of 4,096, its 64 count groups and the launch that adds counts up (beyond 256
+tiles), the run outputs' tiles of 4,096 positions and 64 of them looked back
+over at a time; with keys whose
 digits pile up in one bin, all equal (one run over every tile), descending, or
 spread over all 64 bits."""
 import ctypes
@@ -54,7 +55,7 @@ def test_int32_keys(n):
 @pytest.mark.parametrize("kind", ["table", "wide", "one", "descending", "hot"])
 @pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1023, 1024, 1025, TILE - 1, TILE, TILE + 1, 2 * TILE - 1, 2 * TILE,
                                2 * TILE + 1, 3 * TILE + 17, 16 * TILE, 16 * TILE + 1025, 63 * TILE + 1, 64 * TILE,
-                               65 * TILE + 5, 128 * TILE, 128 * TILE + 1, 300 * TILE + 9])
+                               65 * TILE + 5, 128 * TILE, 128 * TILE + 1, 256 * TILE, 256 * TILE + 1, 300 * TILE + 9])
 def test_dedup_equals_numpy(kind, n):
     if n > 65 * TILE + 5 and kind in ("wide", "descending"):
         n = 129 * TILE + 3
@@ -79,7 +80,7 @@ def test_dedup_equals_numpy(kind, n):
 
 
 @pytest.mark.parametrize("kind", ["table", "wide", "hot"])
-@pytest.mark.parametrize("n", [4097, 6143, 6144, 6145, 8191, 131072, 131073, 262144 - 2048, 262143, 262144, 262145, 266241])
+@pytest.mark.parametrize("n", [4097, 6143, 6144, 6145, 8191, 131072, 131073, 229376 - 2048, 229375, 229376, 229377, 233473, 262144])
 def test_two_round_tiles(kind, n):
     test_dedup_equals_numpy(kind, n)
 
@@ -87,7 +88,7 @@ def test_two_round_tiles(kind, n):
 def test_workspace_of_more_keys_serves_fewer():
     """A workspace sized for n keys is taken for every smaller batch, also across a change of tile size."""
     need, last = ctypes.c_uint64(), 0
-    for n in [1, 4096, 4097, 8192, 131072, 262143, 262144, 262145, 262200, 280000, 524288, 600000]:
+    for n in [1, 4096, 4097, 8192, 131072, 229375, 229376, 229377, 229400, 240000, 262144, 458752, 524288, 600000]:
         _lib.call("nve_amd_dedup_workspace_size", n, ctypes.byref(need))
         assert need.value >= last, n
         last = need.value
