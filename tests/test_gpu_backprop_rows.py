@@ -59,3 +59,25 @@ def test_rows_of_every_position(n, wide, kind, pooling):
     ruq, rout = O.pooling_backprop(keys, pooling, O.CSR, off, off.size - 1, 0, w, O.F32, g, O.F32, 20)
     assert np.array_equal(uq, ruq)
     assert np.array_equal(out, rout.view(np.uint32))
+
+
+@pytest.mark.parametrize("pooling", [O.SUM, O.WMEAN])
+@pytest.mark.parametrize("n,wide", [(200001, False), (262145, False), (600000, False), (1060000, False), (270000, True)])
+def test_rows_of_many_tiles(n, wide, pooling):
+    """A counting workgroup finds the rows of several tiles, of 2,048 and of 4,096 keys, and a first pass over either
+    (behind the launch that adds counts up at 1,060,000 keys) carries them: bags over several tiles, thousands of
+    empty ones between two keys, keys outside every bag."""
+    rng = np.random.default_rng(n + pooling)
+    cut = np.sort(np.concatenate([rng.integers(5000, n - 3000, size=n // 40), np.full(30000, 7 * TILE + 5),
+                                  np.full(3000, 64 * TILE // 2 - 1)]))
+    cut = cut[(cut < 20 * TILE) | (cut > 27 * TILE + 9)]  # a bag of seven tiles
+    off = cut.astype(np.int64)
+    keys = (rng.zipf(1.2, size=n) % 50000).astype(np.int64)
+    if wide:
+        keys = keys * (1 << 30) - (1 << 40)
+    w = rng.uniform(0.1, 1.0, size=n).astype(np.float32) if pooling == O.WMEAN else None
+    g = rng.normal(0, 1, size=(off.size - 1, 4)).astype(np.float32)
+    uq, out = gpu_backprop(keys, pooling, O.CSR, off, 0, w, O.F32, g, O.F32, 4)
+    ruq, rout = O.pooling_backprop(keys, pooling, O.CSR, off, off.size - 1, 0, w, O.F32, g, O.F32, 4)
+    assert np.array_equal(uq, ruq)
+    assert np.array_equal(out, rout.view(np.uint32))
