@@ -10,7 +10,9 @@
 // over a linear table (GPULayer, gpu_embedding_layer.cu:153-189).
 //
 // A row's value area is cut into slices of VB bytes, one per lane of a G-lane
-// group (G = 8..64).  VB is 16 wherever 8 lanes have that much each, also for
+// group (G = 8..64).  VB is 16 for fp16 / fp32 rows past 64 bytes, for byte rows of
+// 65 to 512 bytes 8 where a group has the bag to itself (a byte widens to a value,
+// so that a 16-byte slice is 16 of them), 8 or 4 for narrower rows; also for
 // rows at any alignment (odd widths, quantized rows with their scale behind
 // the values): gfx950 loads 16 bytes from any address, and the last slice of a
 // width that is no multiple of VB starts VB bytes before the end, so it
@@ -18,29 +20,32 @@
 // bits) and no lane reads outside the row.  Rows wider than 64 slices take one
 // workgroup column (blockIdx.y) per 64 slices.
 //
-// Bound: the lines moved between L2 and the CUs at about 10-15 TB/s (random
-// 200-byte rows touch 2.6 lines of 128 bytes), before that the latency of few
+// Bound: wide rows of few distinct lines by the lines moved between L2 and the
+// CUs (random 200-byte rows touch 2.6 lines of 128 bytes: 12 TB/s by lines in
+// 13.5 us; 26 tables as below 12 TB/s), 132-byte int8 rows (2.0 lines, 8 TB/s) by the
+// instructions that widen and broadcast, small launches by the latency of few
 // waves.  Measured against loads as narrow as the row's own alignment
 // (pool_kernel): 16,384 bags of ~30 weighted 200-byte fp16 rows 20.9 -> 13.5 us
 // (8-byte loads, 25 of 32 lanes before), the same bags of 132-byte int8 rows
 // 23.4 -> 15.9 us (4-byte loads and a scale load per lane and row before),
-// 26 tables of 8,192 bags of ~20 256-byte rows 112 -> 101 us; 64 to 16,384 bags
-// over widths of 16 to 768 values 1.56 times as fast for fp16 / fp32 rows and
-// 1.75 times for quantized ones (geometric means).
+// 26 tables of 8,192 bags of ~20 256-byte rows 112 -> 101 us.
 //
-// Same decomposition and summation order as pool_kernel's paths, so for the
-// same lane groups the two produce the same bits: a long bag cut into gpb
+// Same decomposition and summation order as pool_kernel's paths, so where both cut
+// a row into the same lane groups and a bag into the same chunks (fp16 / fp32 rows
+// of whole 16-byte slices) the two produce the same bits: a long bag cut into gpb
 // contiguous key chunks, one chunk per G-lane group, each group accumulating
 // its chunk in key order; an xor butterfly inside each wave; the waves'
-// partial rows added in wave order through LDS.  What is leaner:
-//  * row indices travel between lanes as 32 bits and by VALU lane moves, not
-//    LDS permutes: DPP row_newbcast inside a 16-lane row, v_permlane16_swap /
-//    v_permlane32_swap across rows (gfx950), v_readlane for a whole-wave
-//    group; the address is formed by the consuming lane;
+// partial rows added in wave order through LDS.  A bag that one group adds has
+// the bits of its key order in either.  What is leaner:
+//  * the lane that resolves a key forms its row's address; both halves travel by
+//    one DPP row_newbcast each, inside the 16 lanes of a row, which is why the rows
+//    of a wider group resolve the same 16 keys (over a cache, where a probe is
+//    dear, each its own: spread_keys);
 //  * a quantized row's scale and offset are loaded once per key, by the lane
 //    that resolves the key, and travel the same way;
-//  * the butterfly uses the same lane moves: a + (a of lane l ^ m), formed as
-//    the sum of the two swapped halves, which is the same float addition;
+//  * the butterfly uses DPP row_ror and v_permlane16_swap / v_permlane32_swap
+//    (gfx950): a + (a of lane l ^ m), formed as the sum of the two swapped
+//    halves, which is the same float addition;
 //  * G, VB and the weighting fixed at compile time;
 //  * the cross-wave sum is unrolled so its LDS reads are all in flight.
 #pragma once
@@ -187,7 +192,8 @@ struct LaneKey {
 template <int G>
 constexpr int kRound = G < 16 ? G : 16;
 
-// U keys of a round, from its key J0 on, after their broadcast.
+// U keys of a round, from its key J0 on, after their broadcast.  EARLY: their
+// metadata too, which the lane that resolved the key has loaded.
 template <int SDT, int U, bool W>
 struct BatchKeys {
   uint64_t addr[U];
@@ -201,7 +207,7 @@ __device__ __forceinline__ float group_bcastf(float v) {
   return __uint_as_float(group_bcast<G, J>(__float_as_uint(v)));
 }
 
-template <int SDT, int K, int U, bool W, int J0, int u = 0>
+template <int SDT, int K, int U, bool W, bool EARLY, int J0, int u = 0>
 __device__ __forceinline__ void group_bcast_batch(const LaneKey& k, BatchKeys<SDT, U, W>& b) {
   if constexpr (u < U) {
     static_assert(J0 + u < K, "broadcast source outside the group");
@@ -215,14 +221,14 @@ __device__ __forceinline__ void group_bcast_batch(const LaneKey& k, BatchKeys<SD
       b.w[u] = group_bcastf<K, J0 + u>(k.w);
       b.ws[u] = group_bcastf<K, J0 + u>(k.ws);
     }
-    if constexpr (Fmt<SDT>::meta != 0) {
+    if constexpr (Fmt<SDT>::meta != 0 && EARLY) {
       b.m[u].s = group_bcastf<K, J0 + u>(k.m.s);
       if constexpr (SDT == kQU8F32 || SDT == kXI8AF32 || SDT == kQU8F16)
         b.m[u].o = group_bcastf<K, J0 + u>(k.m.o);
       else
         b.m[u].o = 0.0f;
     }
-    group_bcast_batch<SDT, K, U, W, J0, u + 1>(k, b);
+    group_bcast_batch<SDT, K, U, W, EARLY, J0, u + 1>(k, b);
   }
 }
 
@@ -254,15 +260,19 @@ __device__ __forceinline__ void add_slice(float (&acc)[E], const Vec<VB>& v, con
 }
 
 // The rows of U keys of a round, from its key J0 on: every load in flight, then
-// added in key order.
-template <int SDT, int VB, int K, int U, bool W, int J0>
-__device__ __forceinline__ void add_batch(const LaneKey& k, uint32_t off, float (&acc)[VB / Fmt<SDT>::esize],
+// added in key order.  value_bytes: the place of the metadata in a row.
+template <int SDT, int VB, int K, int U, bool W, bool EARLY, int J0>
+__device__ __forceinline__ void add_batch(const LaneKey& k, uint32_t off, uint32_t value_bytes, float (&acc)[VB / Fmt<SDT>::esize],
                                           float& wsum) {
   BatchKeys<SDT, U, W> b;
-  group_bcast_batch<SDT, K, U, W, J0>(k, b);
+  group_bcast_batch<SDT, K, U, W, EARLY, J0>(k, b);
   Vec<VB> v[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) v[u] = load_slice<VB>(b.addr[u] + off);
+  for (int u = 0; u < U; ++u) {
+    v[u] = load_slice<VB>(b.addr[u] + off);
+    // the zero row has zeros behind its kZeroRowBytes too
+    if constexpr (Fmt<SDT>::meta != 0 && !EARLY) b.m[u] = load_meta_any<SDT>(b.addr[u] + value_bytes);
+  }
   __builtin_amdgcn_sched_barrier(0);  // no addition moves up between the loads
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -503,7 +513,7 @@ __global__ __launch_bounds__(1024) void pool_split_kernel(
     // an immediate source lane)
     auto batch = [&](auto jc) {
       constexpr int j0 = decltype(jc)::value;
-      if (j0 < n) add_batch<SDT, VB, K, U, W, j0 % K>(part[j0 / K], sl.off, acc, wsum);
+      if (j0 < n) add_batch<SDT, VB, K, U, W, true, j0 % K>(part[j0 / K], sl.off, value_bytes, acc, wsum);
     };
     for_batches<U, 0, R / U>(batch);
   }
@@ -641,7 +651,7 @@ struct ShortArgsMT : ShortArgs {
   uint32_t table_rows[kMaxPoolTables];
 };
 
-template <int SDT, int VB, int G, bool W, bool MT, int U>
+template <int SDT, int VB, int G, bool W, bool MT, int U, bool EARLY>
 __global__ __launch_bounds__(256) void pool_short_kernel(std::conditional_t<MT, ShortArgsMT, ShortArgs> a) {
   constexpr int ES = Fmt<SDT>::esize;
   constexpr int E = VB / ES;
@@ -704,7 +714,7 @@ __global__ __launch_bounds__(256) void pool_short_kernel(std::conditional_t<MT, 
     if ((uint64_t)r.key < num_rows) {  // keys outside the table read nothing
       lk.addr = table + (uint64_t)(uint32_t)r.key * rb32;
       lk.w = r.w;
-      if constexpr (Fmt<SDT>::meta != 0) lk.m = load_meta_any<SDT>(lk.addr + value_bytes);
+      if constexpr (Fmt<SDT>::meta != 0 && EARLY) lk.m = load_meta_any<SDT>(lk.addr + value_bytes);
     }
     return lk;
   };
@@ -718,7 +728,7 @@ __global__ __launch_bounds__(256) void pool_short_kernel(std::conditional_t<MT, 
     const int n = (int)((e - k0) < K ? (e - k0) : K);
     auto batch = [&](auto jc) {
       constexpr int j0 = decltype(jc)::value;
-      if (j0 < n) add_batch<SDT, VB, K, U, W, j0>(lk, sl.off, acc, wsum);
+      if (j0 < n) add_batch<SDT, VB, K, U, W, EARLY, j0>(lk, sl.off, value_bytes, acc, wsum);
     };
     for_batches<U, 0, K / U>(batch);
     lk = next;
@@ -803,21 +813,30 @@ hipError_t launch_short_g(const PoolLaunch& a, const PoolSlices& g, hipStream_t 
   const dim3 block(256);
   // 4 rows in flight per lane where more waves wait than the chip holds: the
   // registers of 8 or 16 rows would keep waves out (26 tables of 8,192 bags of
-  // ~20 keys: 4 -> 104 us, 8 -> 111 us).  Launches of at most 4 waves per SIMD
-  // lose none to 8 rows (16,384 bags of ~30 200-byte rows: 13.9 -> 13.6 us),
-  // and bags past 48 keys keep 16 (8 where a lane decodes 16 values or a round has 8 keys).
+  // ~20 keys: 4 -> 104 us, 8 -> 111 us).  Launches of at most 4 waves per SIMD lose none
+  // to 8 rows (16,384 bags of ~30 200-byte rows: 13.9 -> 13.6 us), and bags past 48 keys
+  // keep 16 (8 where a lane decodes 16 values or a round has 8 keys).
+  // A row's metadata is loaded with the row, by every lane.  Loaded a round ahead by
+  // the lane that resolves the key it takes a lane move instead, which saves 3 to 5 %
+  // while the rows stay in the caches (1,024 bags of ~20 132-byte rows 5.5 and 5.3 us),
+  // but its line has to come twice where they do not (uniform keys over 1 M rows,
+  // 8,192 bags of ~30 14.4 and 16.2 us, 32,768 bags 43.3 and 58.6).
   const int64_t avg = a.keys_per_bag > 0 ? a.keys_per_bag
                                          : a.num_keys / (a.num_bags > 0 ? a.num_bags : 1);
   const bool few = (int64_t)grid.x * grid.y * grid.z <= 4 * 256;  // workgroups of a wave per SIMD
+  constexpr bool kMeta = Fmt<SDT>::meta != 0;
+  const bool early = kMeta && (uint64_t)a.num_keys <= (24u << 20) / a.src.row_bytes;
   constexpr int kWide = VB / Fmt<SDT>::esize > 8 || kRound<G> < 16 ? 8 : 16;
-#define NVE_LAUNCH_SHORT(W, U) \
-  hipLaunchKernelGGL((pool_short_kernel<SDT, VB, G, W, MT, U>), grid, block, 0, stream, s)
+#define NVE_LAUNCH_SHORT(W, U, EARLY) \
+  hipLaunchKernelGGL((pool_short_kernel<SDT, VB, G, W, MT, U, EARLY>), grid, block, 0, stream, s)
   if (avg > 48) {
-    if (a.weighted) NVE_LAUNCH_SHORT(true, kWide); else NVE_LAUNCH_SHORT(false, kWide);
+    if (a.weighted) NVE_LAUNCH_SHORT(true, kWide, false); else NVE_LAUNCH_SHORT(false, kWide, false);
+  } else if (few && early) {
+    if (a.weighted) NVE_LAUNCH_SHORT(true, 8, kMeta); else NVE_LAUNCH_SHORT(false, 8, kMeta);
   } else if (few) {
-    if (a.weighted) NVE_LAUNCH_SHORT(true, 8); else NVE_LAUNCH_SHORT(false, 8);
+    if (a.weighted) NVE_LAUNCH_SHORT(true, 8, false); else NVE_LAUNCH_SHORT(false, 8, false);
   } else {
-    if (a.weighted) NVE_LAUNCH_SHORT(true, 4); else NVE_LAUNCH_SHORT(false, 4);
+    if (a.weighted) NVE_LAUNCH_SHORT(true, 4, false); else NVE_LAUNCH_SHORT(false, 4, false);
   }
 #undef NVE_LAUNCH_SHORT
   return hipGetLastError();

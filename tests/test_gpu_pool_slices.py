@@ -163,3 +163,16 @@ def test_bags_of_a_few_dozen_keys(dtype, count, bags, pooling, whole):
     the oracle bit for bit, one that is cut stays within the tolerance of its order."""
     lens = np.random.default_rng(bags).integers(25, 70, size=bags)
     check(dtype, count, pooling, lens, 1, whole, bags + count)
+
+
+@pytest.mark.parametrize("lens,bags", [((0, 5), 3000), ((10, 40), 8192), ((8, 20), 33000), ((50, 70), 8192)],
+                         ids=["up_to_4_keys", "more_bytes", "more_waves", "past_48_keys"])
+@pytest.mark.parametrize("dtype,count", [(t, d) for t in (O.QI8_F32, O.QI8_F16, O.QU8_F32, O.QU8_F16, O.XI8A_F32, O.XE4M3_F32)
+                                         for d in (130, 514)] + [(O.F16, 66)])
+def test_metadata_loaded_with_the_row(dtype, count, lens, bags):
+    """Launches whose rows pass the size up to which metadata is loaded ahead, in every number of rows in flight; keys
+    outside the table and slots past the end of a bag read the zero row's metadata."""
+    if count == 514:
+        bags //= 4
+    lens = np.random.default_rng(bags).integers(lens[0], lens[1], size=bags)
+    check(dtype, count, _lib.POOL_WSUM, lens, 1, lens.mean() < 50 or count != 514, bags + count)
