@@ -813,9 +813,11 @@ hipError_t launch_short_g(const PoolLaunch& a, const PoolSlices& g, hipStream_t 
   const dim3 block(256);
   // 4 rows in flight per lane where more waves wait than the chip holds: the
   // registers of 8 or 16 rows would keep waves out (26 tables of 8,192 bags of
-  // ~20 keys: 4 -> 104 us, 8 -> 111 us).  Launches of at most 4 waves per SIMD lose none
-  // to 8 rows (16,384 bags of ~30 200-byte rows: 13.9 -> 13.6 us), and bags past 48 keys
-  // keep 16 (8 where a lane decodes 16 values or a round has 8 keys).
+  // ~20 keys: 4 -> 104 us, 8 -> 111 us), and for bags of up to 4 keys, whose other
+  // rows would be zero rows (16,384 bags of 2 256-byte rows: 4 -> 2.96 us, 8 -> 3.31).
+  // Other launches of at most 4 waves per SIMD lose none to 8 rows (16,384 bags of ~30
+  // 200-byte rows: 13.9 -> 13.6 us), and bags past 48 keys keep 16 (8 where a lane
+  // decodes 16 values or a round has 8 keys).
   // A row's metadata is loaded with the row, by every lane.  Loaded a round ahead by
   // the lane that resolves the key it takes a lane move instead, which saves 3 to 5 %
   // while the rows stay in the caches (1,024 bags of ~20 132-byte rows 5.5 and 5.3 us),
@@ -831,9 +833,9 @@ hipError_t launch_short_g(const PoolLaunch& a, const PoolSlices& g, hipStream_t 
   hipLaunchKernelGGL((pool_short_kernel<SDT, VB, G, W, MT, U, EARLY>), grid, block, 0, stream, s)
   if (avg > 48) {
     if (a.weighted) NVE_LAUNCH_SHORT(true, kWide, false); else NVE_LAUNCH_SHORT(false, kWide, false);
-  } else if (few && early) {
+  } else if (few && avg > 4 && early) {
     if (a.weighted) NVE_LAUNCH_SHORT(true, 8, kMeta); else NVE_LAUNCH_SHORT(false, 8, kMeta);
-  } else if (few) {
+  } else if (few && avg > 4) {
     if (a.weighted) NVE_LAUNCH_SHORT(true, 8, false); else NVE_LAUNCH_SHORT(false, 8, false);
   } else {
     if (a.weighted) NVE_LAUNCH_SHORT(true, 4, false); else NVE_LAUNCH_SHORT(false, 4, false);
