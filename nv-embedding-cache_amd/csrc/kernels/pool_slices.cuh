@@ -820,14 +820,15 @@ hipError_t launch_short_g(const PoolLaunch& a, const PoolSlices& g, hipStream_t 
   // decodes 16 values or a round has 8 keys).
   // A row's metadata is loaded with the row, by every lane.  Loaded a round ahead by
   // the lane that resolves the key it takes a lane move instead, which saves 3 to 5 %
-  // while the rows stay in the caches (1,024 bags of ~20 132-byte rows 5.5 and 5.3 us),
-  // but its line has to come twice where they do not (uniform keys over 1 M rows,
-  // 8,192 bags of ~30 14.4 and 16.2 us, 32,768 bags 43.3 and 58.6).
+  // while the rows' lines stay in the caches (1,024 bags of ~20 132-byte rows 5.5 and
+  // 5.3 us, 16,384 bags of 8 6.5 and 5.7), but the last one has to come twice where they
+  // do not (uniform keys over 1 M rows, 8,192 bags of ~30 14.4 and 16.2 us, 32,768 bags
+  // 43.3 and 58.6; 36-byte rows, 32,768 bags of ~20 17.6 and 25.3).
   const int64_t avg = a.keys_per_bag > 0 ? a.keys_per_bag
                                          : a.num_keys / (a.num_bags > 0 ? a.num_bags : 1);
   const bool few = (int64_t)grid.x * grid.y * grid.z <= 4 * 256;  // workgroups of a wave per SIMD
   constexpr bool kMeta = Fmt<SDT>::meta != 0;
-  const bool early = kMeta && (uint64_t)a.num_keys <= (24u << 20) / a.src.row_bytes;
+  const bool early = kMeta && (uint64_t)a.num_keys <= (48u << 20) / (a.src.row_bytes + 127);  // by lines touched
   constexpr int kWide = VB / Fmt<SDT>::esize > 8 || kRound<G> < 16 ? 8 : 16;
 #define NVE_LAUNCH_SHORT(W, U, EARLY) \
   hipLaunchKernelGGL((pool_short_kernel<SDT, VB, G, W, MT, U, EARLY>), grid, block, 0, stream, s)
