@@ -10,6 +10,8 @@ namespace nve_amd {
 // per SIMD of whole bags (131,072 lanes) on, a group per bag is faster: bags of ~35
 // weighted keys over 128-byte rows, 16,384 of them 13.2 and 8.4 us, over 256-byte rows,
 // 8,192 bags 11.8 and 7.4; with half as many bags of ~64 keys unweighted 8.3 and 9.2.
+// Byte rows of 129 to 512 bytes take twice the lanes in whole bags (4,096 bags of ~40
+// weighted 264-byte rows 19.3 and 14.4 us).
 // Groups of 32 lanes cut such a bag in two; with weights and up to 48 keys a group
 // per bag is faster at any number of bags (512-byte rows, ~35 keys, 1,024 bags 7.1 and
 // 5.0 us; 64 bags of ~63 keys 5.3 and 5.9).
@@ -22,12 +24,14 @@ static int slice_groups(const PoolLaunch& a, int g) {
   if (a.force_split != 0 || gpb == 1 || gpb * g > 64) return gpb;
   const int64_t avg = a.keys_per_bag > 0 ? a.keys_per_bag : a.num_keys / a.num_bags;
   const int64_t simd_waves = 1024 * 64;  // lanes of a wave per SIMD
-  const int64_t lanes = a.num_bags * g;
+  const int64_t bytes = a.count * value_elem_bytes(a.stored_dtype);
+  int whole = g;  // lanes of a bag that is not shared: byte rows are then cut finer
+  while (value_elem_bytes(a.stored_dtype) == 1 && whole * 8 < bytes && whole < 64) whole *= 2;
+  const int64_t lanes = a.num_bags * whole;
   if (a.src.cache_data != nullptr) {
-    const uint64_t area = (uint64_t)a.count * value_elem_bytes(a.stored_dtype);
-    const bool wide = ((uint64_t)a.src.table | (uint64_t)a.src.cache_data | a.src.row_bytes | area |
+    const bool wide = ((uint64_t)a.src.table | (uint64_t)a.src.cache_data | a.src.row_bytes | (uint64_t)bytes |
                        (uint64_t)a.out | (uint64_t)a.out_stride) % 16 == 0;
-    const bool many = avg <= 48 && lanes >= (a.weighted && area > 64 ? 2 : 3) * simd_waves;
+    const bool many = avg <= 48 && lanes >= (a.weighted && bytes > 64 ? 2 : 3) * simd_waves;
     return many && wide ? gpb : 64 / g;
   }
   return (avg <= 64 && lanes >= 2 * simd_waves) || (avg <= 48 && g == 32 && a.weighted) ? 1 : 64 / g;

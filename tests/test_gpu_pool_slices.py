@@ -156,7 +156,8 @@ def test_narrow_rows_in_bags_of_a_few_dozen_keys(dtype, count, bags):
 @pytest.mark.parametrize("dtype,count,bags,pooling,whole", [
     (O.F16, 64, 16384, _lib.POOL_WSUM, True), (O.F16, 64, 16383, _lib.POOL_WSUM, False),
     (O.F32, 64, 8192, _lib.POOL_SUM, True), (O.F32, 64, 8191, _lib.POOL_SUM, False),
-    (O.QI8_F32, 130, 8192, _lib.POOL_WMEAN, True), (O.F16, 256, 50, _lib.POOL_WMEAN, True),
+    (O.QI8_F32, 130, 4096, _lib.POOL_WMEAN, True),
+    (O.QI8_F32, 130, 4095, _lib.POOL_WMEAN, False), (O.F16, 256, 50, _lib.POOL_WMEAN, True),
     (O.F16, 256, 50, _lib.POOL_MEAN, False), (O.F16, 256, 4096, _lib.POOL_MEAN, True)])
 def test_bags_of_a_few_dozen_keys(dtype, count, bags, pooling, whole):
     """Bags of 33 to 64 keys on both sides of the lines where a wave shares a bag: one added by a single group equals
@@ -173,6 +174,6 @@ def test_metadata_loaded_with_the_row(dtype, count, lens, bags):
     """Launches whose rows pass the size up to which metadata is loaded ahead, in every number of rows in flight; keys
     outside the table and slots past the end of a bag read the zero row's metadata."""
     if count == 514:
-        bags //= 4
+        bags //= 2
     lens = np.random.default_rng(bags).integers(lens[0], lens[1], size=bags)
     check(dtype, count, _lib.POOL_WSUM, lens, 1, lens.mean() < 50 or count != 514, bags + count)
