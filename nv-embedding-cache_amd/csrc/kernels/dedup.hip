@@ -9,13 +9,13 @@
 // the stable inverse map and exclusive offsets.
 //
 // dedup-then-gather needs no order, so it dedups by hashing instead of
-// sorting (three launches): every distinct key of a workgroup
-// claims a slot of an open-addressed table (linear probing, at most
-// half full) with one compare-and-swap, the winner becoming the key's owner
-// and its workgroup copying the key's table row to the owner's output row at
-// once (each distinct row read once); with 32-bit keys a slot holds key and
-// owner, so every claimant learns the owner at once; then every other
-// position copies its owner's output row (UnpackDedup, cuda_utils.cuh:24-79).
+// sorting (three launches): every distinct key of a workgroup claims a slot of
+// an open-addressed table (linear probing, at most half full) with one
+// compare-and-swap, the winner becoming the key's owner and its workgroup
+// copying the key's table row to the owner's output row at once (each distinct
+// row read once); with 32-bit keys a slot holds key and owner, so every claimant
+// learns the owner at once; then every other position copies its owner's output
+// row (UnpackDedup, cuda_utils.cuh:24-79).
 #include "device_common.cuh"
 #include "dedup_launch.hpp"
 #include "lane_moves.cuh"
