@@ -20,14 +20,15 @@
 // bits) and no lane reads outside the row.  Rows wider than 64 slices take one
 // workgroup column (blockIdx.y) per 64 slices.
 //
-// Bound: wide rows of few distinct lines by the lines moved between L2 and the
-// CUs (random 200-byte rows touch 2.6 lines of 128 bytes: 12 TB/s by lines in
-// 13.5 us; 26 tables as below 12 TB/s), 132-byte int8 rows (2.0 lines, 8 TB/s) by the
-// instructions that widen and broadcast, small launches by the latency of few
-// waves.  Measured against loads as narrow as the row's own alignment
+// Bound: the lines moved into the CUs, in small launches the latency of few waves.
+// The plain read kernel (launch_read_ceiling) takes random 256-byte rows at 16.7
+// TB/s from a table in L2 (4 MB), at 9.3 to 7.3 from the MALL (16 to 200 MB) and at 5.9
+// from HBM (4 GB); batches of Zipf keys lie between the first two: 200-byte rows (2.6
+// lines of 128 bytes) at 12 TB/s by lines, 26 tables as below at 12, 132-byte int8 rows
+// (2.0 lines) at 8.5 (what holds those back has not been taken apart).  Measured against loads as narrow as the row's own alignment
 // (pool_kernel): 16,384 bags of ~30 weighted 200-byte fp16 rows 20.9 -> 13.5 us
 // (8-byte loads, 25 of 32 lanes before), the same bags of 132-byte int8 rows
-// 23.4 -> 15.9 us (4-byte loads and a scale load per lane and row before),
+// 23.6 -> 14.8 us (4-byte loads and a scale load per lane and row before),
 // 26 tables of 8,192 bags of ~20 256-byte rows 112 -> 101 us.
 //
 // Same decomposition and summation order as pool_kernel's paths, so where both cut
