@@ -80,7 +80,8 @@ def test_dedup_equals_numpy(kind, n):
 
 
 @pytest.mark.parametrize("kind", ["table", "wide", "hot"])
-@pytest.mark.parametrize("n", [4097, 6143, 6144, 6145, 8191, 131072, 131073, 229376 - 2048, 229375, 229376, 229377, 233473, 262144])
+@pytest.mark.parametrize("n", [4097, 6143, 6144, 6145, 8191, 131072, 131073, 229376 - 2048, 229375, 229376, 229377, 233473,
+                               262144 - 2048, 262143, 262144, 262145, 266241])
 def test_two_round_tiles(kind, n):
     test_dedup_equals_numpy(kind, n)
 
@@ -88,7 +89,8 @@ def test_two_round_tiles(kind, n):
 def test_workspace_of_more_keys_serves_fewer():
     """A workspace sized for n keys is taken for every smaller batch, also across a change of tile size."""
     need, last = ctypes.c_uint64(), 0
-    for n in [1, 4096, 4097, 8192, 131072, 229375, 229376, 229377, 229400, 240000, 262144, 458752, 524288, 600000]:
+    for n in [1, 4096, 4097, 8192, 131072, 229375, 229376, 229377, 229400, 240000, 262143, 262144, 262145, 262200,
+              280000, 458752, 524288, 600000]:
         _lib.call("nve_amd_dedup_workspace_size", n, ctypes.byref(need))
         assert need.value >= last, n
         last = need.value
